@@ -366,7 +366,7 @@ struct vpfp_plan_s {
   float* dft_mat = nullptr;   // [2][nx][nx] forward and inverse real-DFT matrices
   double tuned_us = 0.0;
   int delta = 0;                 // f stored as f - M(v)
-  double* bg = nullptr;          // M(v_m) [nv] (FP64) and its DFT [nv] (storage precision)
+  double* bg = nullptr;          // M(v_m) [nv] (FP64) and its spectrum tables [nv] (storage precision)
   void* bg_hat = nullptr;
   double *kx = nullptr, *okx = nullptr, *v = nullptr, *kv = nullptr;
   void* tw_v = nullptr;          // cx<T> [lo | hi] tables for nv
@@ -865,7 +865,7 @@ struct vpfp_batch_s {
   vpfc_net_t closure = nullptr;  // learned closure after every step (FP32, nv 256)
   int groups = 0;                // groups holding this batch (vpfp_group_create)
   int delta = 0;                 // f stored as f - M(v)
-  double* bg = nullptr;          // M(v_m) [nv] and its unnormalised DFT [nv]
+  double* bg = nullptr;          // M(v_m) [nv] and its spectrum tables [nv]
   void* bg_hat = nullptr;        // (cx<double> or cx<float>: the storage precision)
   double dv = 0, dt = 0, v0 = 0, dvv = 0, dk_v = 0;
   double *dk_x = nullptr, *okx = nullptr, *nu_dt = nullptr, *v = nullptr;
@@ -1483,8 +1483,10 @@ int autotune_group(vpfp_group_s* g, int n_steps, hipStream_t s) {
 // ====================================================================== C ABI
 namespace {
 
-// unit Maxwellian on a v grid (v_m = v0 + m dvv) and its DFT
-// sum_m M_m exp(-2 pi i k m / N) (direct sum in FP64 with an exact twiddle index)
+// unit Maxwellian on a v grid (v_m = v0 + m dvv) and the spectrum tables of
+// vp::BgPhaseMul from its DFT B_k = sum_m M_m exp(-2 pi i k m / N) (direct sum
+// in FP64 with an exact twiddle index): with W_k = exp(-2 pi i k / N) and
+// M = N / 2, hat[k] = B_k (1 + i conj W_k) / N, hat[M + k] = B_{k+M} (1 - i conj W_k) / N
 void background_tables(int N, double v0, double dvv, std::vector<double>& m, std::vector<cx<double>>& hat) {
   m.assign(N, 0.0);
   for (int i = 0; i < N; ++i) {
@@ -1505,6 +1507,14 @@ void background_tables(int N, double v0, double dvv, std::vector<double>& m, std
       im += m[i] * wi[j];
     }
     hat[k] = vp::mk<double>(re, im);
+  }
+  const int M = N / 2;
+  for (int k = 0; k < M; ++k) {
+    // i conj W_k = (wi, wr): W_k = (wr, wi)
+    const cx<double> p = vp::mk<double>((1.0 + wi[k]) / N, wr[k] / N);
+    const cx<double> m = vp::mk<double>((1.0 - wi[k]) / N, -wr[k] / N);
+    hat[k] = vp::mul(hat[k], p);
+    hat[k + M] = vp::mul(hat[k + M], m);
   }
 }
 

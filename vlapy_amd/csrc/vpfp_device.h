@@ -268,6 +268,37 @@ VP_HD constexpr int brev(int i) {
   return r;
 }
 
+// (a, b) <- (a + W b, a - W b) with W = W_32^J (inverse: its conjugate).  For
+// a W off the axes one of its parts is factored out, W b = c (b' + i b'') with
+// c the larger part, so that c goes into the two sums as their fma: 6
+// instructions instead of the 8 of a product and two sums.
+template <bool INV, class T>
+VP_HD void butterfly(cx<T>& a, cx<T>& b, int J) {
+  J &= 31;
+  if ((J & 7) == 0) {
+    const cx<T> w = tw32<INV>(b, J), x = a;
+    a = add(x, w);
+    b = sub(x, w);
+    return;
+  }
+  const double cd = cos32(J), sd = INV ? -sin32(J) : sin32(J);
+  const bool cbig = (cd < 0 ? -cd : cd) >= (sd < 0 ? -sd : sd);
+  const T f = (T)(cbig ? cd : sd), r = (T)(cbig ? sd / cd : cd / sd);
+  // W b = (b.re c + b.im s, b.im c - b.re s)
+  const bool one = r == T(1), mone = r == T(-1);
+  T u, w;
+  if (cbig) {
+    u = one ? b.re + b.im : mone ? b.re - b.im : b.re + r * b.im;
+    w = one ? b.im - b.re : mone ? b.im + b.re : b.im - r * b.re;
+  } else {
+    u = b.im + r * b.re;
+    w = r * b.im - b.re;
+  }
+  const cx<T> x = a;
+  a = mk<T>(x.re + f * u, x.im + f * w);
+  b = mk<T>(x.re - f * u, x.im - f * w);
+}
+
 template <int R, bool INV, class T>
 VP_HD void dft(cx<T>* x) {
   static_assert(R >= 1 && R <= 32 && (R & (R - 1)) == 0, "radix must be a power of two <= 32");
@@ -280,12 +311,7 @@ VP_HD void dft(cx<T>* x) {
 #pragma unroll
     for (int g = 0; g < R; g += 2 * h) {
 #pragma unroll
-      for (int j = 0; j < h; ++j) {
-        const cx<T> a = y[g + j];
-        const cx<T> b = tw32<INV>(y[g + j + h], j * (16 / h));
-        y[g + j] = add(a, b);
-        y[g + j + h] = sub(a, b);
-      }
+      for (int j = 0; j < h; ++j) butterfly<INV>(y[g + j], y[g + j + h], j * (16 / h));
     }
   }
 #pragma unroll
@@ -341,16 +367,21 @@ VP_HD void tw_stage(Ctx& c, cx<T>* dst, const cx<T>* src) {
 // Register layout: thread t holds element t + i*TPT in v[i], i < Q = M/TPT.
 // A pass of radix R with NS = product of the earlier radices takes the
 // butterfly j = t + q*TPT (inputs j + r*M/R = v[q + r*Q/R]), twiddles input r
-// by W_{NS*R}^{r*(j mod NS)}, does an R-point DFT and writes output r to
-// position (j - j mod NS)*R + j mod NS + r*NS.  After the last pass the data
-// are in natural order, both in v and in `buf`.
+// by W_{NS*R}^{r*(j mod NS)}, does an R-point DFT and sends output r to
+// position (j - j mod NS)*R + j mod NS + r*NS.  In the last pass NS = M/R, so
+// j mod NS = j and output r belongs at j + r*M/R: the place its register
+// already has.  Only the passes before the last go through `buf`; the
+// transform ends with the data in natural order in v and `buf` free.
 //
 // tw(n) = exp(-2 pi i n / (2M)); the M-point twiddle W_M^n is tw(2n).
 // ---------------------------------------------------------------------------
 // `act` false: the thread only takes part in the barriers (no LDS writes).
-template <class T, int M, int TPT, int R, int NS, bool INV, class TW, class Ctx>
-VP_HD void st_pass(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, bool act) {
+template <class T, int M, int TPT, bool INV, int NS = 1, class TW, class Ctx>
+VP_HD void fft(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, bool act = true) {
   constexpr int Q = M / TPT;
+  static_assert(Q >= 2 && Q * TPT == M, "each thread must hold at least two values");
+  constexpr int RMAX = Q < 16 ? Q : 16;
+  constexpr int R = (M / NS) < RMAX ? (M / NS) : RMAX;
   constexpr int NB = Q / R;
   static_assert(NB * R == Q, "radix must divide the per-thread count");
 #pragma unroll
@@ -368,26 +399,24 @@ VP_HD void st_pass(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, bool act) 
       }
     }
     dft<R, INV>(u);
-    const int base = (j - k) * R + k;
-    if (act) {
+    if constexpr (NS * R < M) {
+      if (act) {
+        const int base = (j - k) * R + k;
 #pragma unroll
-      for (int r = 0; r < R; ++r) buf[pidx(base + r * NS)] = u[r];
+        for (int r = 0; r < R; ++r) buf[pidx(base + r * NS)] = u[r];
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q + r * NB] = u[r];
     }
   }
-  c.sync();
+  if constexpr (NS * R < M) {
+    c.sync();
 #pragma unroll
-  for (int i = 0; i < Q; ++i) v[i] = buf[pidx(t + i * TPT)];
-  c.sync();
-}
-
-template <class T, int M, int TPT, bool INV, int NS = 1, class TW, class Ctx>
-VP_HD void fft(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, bool act = true) {
-  constexpr int Q = M / TPT;
-  static_assert(Q >= 2 && Q * TPT == M, "each thread must hold at least two values");
-  constexpr int RMAX = Q < 16 ? Q : 16;
-  constexpr int R = (M / NS) < RMAX ? (M / NS) : RMAX;
-  st_pass<T, M, TPT, R, NS, INV>(c, v, buf, tw, t, act);
-  if constexpr (NS * R < M) fft<T, M, TPT, INV, NS * R>(c, v, buf, tw, t, act);
+    for (int i = 0; i < Q; ++i) v[i] = buf[pidx(t + i * TPT)];
+    c.sync();
+    fft<T, M, TPT, INV, NS * R>(c, v, buf, tw, t, act);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -398,35 +427,51 @@ VP_HD void fft(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, bool act = tru
 // of the multiplier, which is what taking Re() of the complex inverse leaves).
 // ---------------------------------------------------------------------------
 
+// s (C + i S) / (C^2 + S^2), with the rounding error of the norm taken to first
+// order.  A spectrum with F_{k+M} = 0 (a resolved f) comes out of the
+// expression below times (C - i S) (C + i S) / M: dividing by the rounded
+// norm keeps the pushers from scaling every mode by the same rounding error
+// step after step, and what is left of the error of C and S is one of P_M.
+VP_HD float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
+VP_HD double fma_t(double a, double b, double c) { return fma(a, b, c); }
+template <class T>
+VP_HD cx<T> half_phase(T C, T S, T s) {
+  const T e = C * C > T(0.5) ? fma_t(S, S, fma_t(C, C, T(-1))) : fma_t(C, C, fma_t(S, S, T(-1)));
+  const T w = s - s * e;
+  return mk<T>(C * w, S * w);
+}
+
 // Phase shift exp(-i theta_k) of the exponential pushers, theta_k = k phi
 // with phi = (dk * dt) * s: dk is the first wavenumber of an fftfreq table
 // (checked on the host to be linear in k to rounding), s the advection speed
-// (e(x) for the v-kick, v for the x-drift).  Bins are visited in the order
-// k = t, t + TPT, t + 2 TPT, ... so P_k is a running product; the partner
-// phase is P_{M-k} = exp(-i theta_M) conj(P_k).
+// (e(x) for the v-kick, v for the x-drift).
+//
+// With P_{M-k} = P_M conj(P_k) the unpack, multiply and repack of couple()
+// below collapse into one expression in Z_k and Z_{M-k}:
+//   Z'_k = p_k [ (C + i S sin(pi k / M)) Z_k + S cos(pi k / M) conj(Z_{M-k}) ],
+//   C + i S = exp(i M phi / 2),  p_k = exp(-i (k - M/2) phi) / M,
+// for 0 < k < M (from E + i O = Z and W O + i conj(W) E =
+// -sin Z + i cos conj(Z_{M-k}) with W = exp(-i pi k / M)); the DC bin keeps its
+// value and the Nyquist bin gets cos(M phi) = 1 - 2 S^2.  16 instructions per
+// bin instead of 44 for the three steps apart; with the last Stockham passes
+// kept in registers: nv = 8192 FP64 kicks 69 -> 63 us (1024 rows), nx = 1024
+// FP64 drift 66 -> 59 us, nx = 128 FP32 drift of a scan 503 -> 482 us.  Bins
+// are visited in the order k = t, t + TPT, ..., so p_k is a running product.
 template <class T>
 struct PhaseMul {
-  static constexpr bool kBg = false;
-  cx<T> cur, step, pm;
+  T C, S;
+  cx<T> cur, step;
   VP_HD PhaseMul(double phi, int M, int t, int TPT) {
-    cis_neg((double)M * phi, pm);
+    cx<T> h;
+    cis_neg(-0.5 * (double)M * phi, h);
+    C = h.re;
+    S = h.im;
     cis_neg((double)t * phi, cur);
+    cur = mul(cur, half_phase(C, S, T(1) / T(M)));
     cis_neg((double)TPT * phi, step);
-  }
-  VP_HD void pair(int k, cx<T>& pk, cx<T>& pmk) {
-    if (k == 0) {
-      pk = mk<T>(T(1), T(0));
-      pmk = mk<T>(pm.re, T(0));
-    } else {
-      pk = cur;
-      pmk = mulc(pm, pk);
-    }
-    cur = mul(cur, step);
   }
 };
 
-// Poisson multiplier i * one_over_kx (zero real part at DC and Nyquist);
-// okx is an LDS copy of the one_over_kx table.
 // exp(-i theta) - 1 without cancellation: (-2 sin^2(theta/2), -2 sin(theta/2)
 // cos(theta/2)), from one sincos of the half angle after reduction in double
 // (FP32 sincos for FP32 results: both parts keep FP32 relative precision
@@ -445,55 +490,35 @@ VP_HD cx<T> cis_neg_m1(double th) {
   }
 }
 
-// PhaseMul on a stored deviation f - B from a fixed background B whose
-// unnormalised spectrum is bhat [N] (storage precision): the shift of B itself
-// enters as F'_k += bhat_k (P_k - 1), F'_{k+M} += bhat_{k+M} (conj P_{M-k} - 1).
-// c_k = P_k - 1 is carried by c_{k+s} = c_k + c_s + c_k c_s (no cancellation
-// for small shifts) and the phases themselves are P_k = 1 + c_k,
-// P_M = conj(1 + cpm) with cpm = exp(+i M phi) - 1.  couple() calls init()
-// once, then pair(k, ...) and bg_add(k, ...) for each k in turn; all of the
-// state is formed in init(), after the forward transform.
+// PhaseMul on a stored deviation f - B from a fixed background B with
+// unnormalised spectrum B_k: the shift of B itself enters as
+// F'_k += B_k (P_k - 1), F'_{k+M} += B_{k+M} (conj P_{M-k} - 1), in the repacked
+// spectrum
+//   Z'_k += b1_k (P_k - 1) + b2_k (conj P_{M-k} - 1),
+//   b1_k = B_k (1 + i conj W_k) / N,  b2_k = B_{k+M} (1 - i conj W_k) / N,
+// tables the host forms ([b1: M | b2: M], storage precision).  c_k = P_k - 1 is
+// carried by c_{k+s} = c_k + c_s + c_k c_s (no cancellation for small shifts);
+// the data's phases are p_k = (1 + c_k) (C + i S) / M.
 template <class T>
 struct BgPhaseMul {
-  static constexpr bool kBg = true;
-  double phi;
-  int M, t, TPT;
-  const cx<T>* bhat;
+  T C, S;
   cx<T> cm, cs, cpm;  // P_k - 1, P_TPT - 1, exp(+i M phi) - 1
-  VP_HD BgPhaseMul(double phi_, int M_, int t_, int TPT_, const cx<T>* bhat_)
-      : phi(phi_), M(M_), t(t_), TPT(TPT_), bhat(bhat_) {}
-  VP_HD void init() {
+  const cx<T>* bhat;
+  VP_HD BgPhaseMul(double phi, int M, int t, int TPT, const cx<T>* bhat_) : bhat(bhat_) {
+    cx<T> h;
+    cis_neg(-0.5 * (double)M * phi, h);
+    C = h.re;
+    S = h.im;
+    cpm = mk<T>(T(-2) * S * S, T(2) * S * C);
     cm = cis_neg_m1<T>((double)t * phi);
     cs = cis_neg_m1<T>((double)TPT * phi);
-    cpm = cis_neg_m1<T>(-(double)M * phi);
-  }
-  VP_HD void pair(int k, cx<T>& pk, cx<T>& pmk) {
-    const cx<T> pm = mk<T>(T(1) + cpm.re, -cpm.im);
-    if (k == 0) {
-      pk = mk<T>(T(1), T(0));
-      pmk = mk<T>(pm.re, T(0));
-    } else {
-      pk = mk<T>(T(1) + cm.re, cm.im);
-      pmk = mulc(pm, pk);
-    }
-  }
-  VP_HD void bg_add(int k, cx<T>& G1, cx<T>& G2) {
-    const cx<T> B1 = bhat[k], B2 = bhat[k + M];
-    if (k == 0) {
-      // DC unchanged; Nyquist multiplier Re(P_M) = cos(M phi)
-      G2 = add(G2, mk<T>(B2.re * cpm.re, B2.im * cpm.re));
-    } else {
-      G1 = add(G1, mul(B1, cm));
-      const cx<T> q = add(add(cpm, cm), mul(cpm, cm));
-      G2 = add(G2, mul(B2, q));
-    }
-    cm = add(add(cm, cs), mul(cm, cs));
   }
 };
 
+// Poisson multiplier i * one_over_kx (zero real part at DC and Nyquist);
+// okx is an LDS copy of the one_over_kx table.
 template <class T>
 struct PoissonMul {
-  static constexpr bool kBg = false;
   const double* okx;
   int M;
   VP_HD void pair(int k, cx<T>& pk, cx<T>& pmk) {
@@ -514,12 +539,11 @@ struct PoissonMul {
 // the repacked spectrum Z'_k = (F'_k + F'_{k+M} + i (F'_k - F'_{k+M}) conj W)/N
 // inverse-transforms (unnormalised M-point) to f'_{2j} + i f'_{2j+1}.
 // v[i] holds Z_k and pz[i] holds Z_{M-k} for k = t + i*TPT; tw(k) = W^k.
-template <class T, int M, int TPT, class Mul, class TW>
-VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, Mul& mult) {
+template <class T, int M, int TPT, class TW>
+VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, PoissonMul<T>& mult) {
   constexpr int Q = M / TPT;
   const T invN = T(1) / T(2 * M);
   const T h = T(0.5);
-  if constexpr (Mul::kBg) mult.init();
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
     const int k = t + i * TPT;
@@ -531,12 +555,63 @@ VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, Mul& mult) {
     const cx<T> Fk = add(E, WO), Fkm = sub(E, WO);
     cx<T> pk, pmk;
     mult.pair(k, pk, pmk);
-    cx<T> G1 = mul(pk, Fk);
-    cx<T> G2 = mulc(Fkm, pmk);
-    if constexpr (Mul::kBg) mult.bg_add(k, G1, G2);
+    const cx<T> G1 = mul(pk, Fk);
+    const cx<T> G2 = mulc(Fkm, pmk);
     const cx<T> S = add(G1, G2);
     const cx<T> D = mulc(sub(G1, G2), W);
     v[i] = mk<T>((S.re - D.im) * invN, (S.im + D.re) * invN);
+  }
+}
+
+// (C + i S sin) a + S cos conj(p), W = (cos, -sin)
+template <class T>
+VP_HD cx<T> couple_bin(T C, T S, cx<T> W, cx<T> a, cx<T> p) {
+  const T g = S * W.im, h = S * W.re;  // g = -S sin
+  return mk<T>(C * a.re + g * a.im + h * p.re, C * a.im - g * a.re - h * p.im);
+}
+
+// DC unchanged, Nyquist times 1 + nyq
+template <class T>
+VP_HD cx<T> couple_dc(cx<T> a, T nyq, T invN) {
+  const T f0 = a.re + a.im, fm = a.re - a.im;
+  const T g2 = fm + nyq * fm;
+  return mk<T>((f0 + g2) * invN, (f0 - g2) * invN);
+}
+
+template <class T, int M, int TPT, class TW>
+VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, PhaseMul<T>& m) {
+  constexpr int Q = M / TPT;
+  cx<T> cur = m.cur;
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    const cx<T> a = v[i];
+    v[i] = mul(cur, couple_bin(m.C, m.S, tw(t + i * TPT), a, pz[i]));
+    if (i == 0 && t == 0) v[0] = couple_dc(a, T(-2) * m.S * m.S, T(1) / T(2 * M));
+    if (i + 1 < Q) cur = mul(cur, m.step);
+  }
+}
+
+template <class T, int M, int TPT, class TW>
+VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, BgPhaseMul<T>& m) {
+  constexpr int Q = M / TPT;
+  const cx<T> kap = half_phase(m.C, m.S, T(1) / T(M));
+  cx<T> cm = m.cm;
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    const int k = t + i * TPT;
+    const cx<T> B1 = m.bhat[k], B2 = m.bhat[k + M];
+    const cx<T> a = v[i];
+    const cx<T> pk = mk<T>(kap.re + (kap.re * cm.re - kap.im * cm.im), kap.im + (kap.re * cm.im + kap.im * cm.re));
+    const cx<T> q = mk<T>((m.cpm.re + cm.re) + (m.cpm.re * cm.re - m.cpm.im * cm.im),
+                          (m.cpm.im + cm.im) + (m.cpm.re * cm.im + m.cpm.im * cm.re));
+    const cx<T> y = mul(pk, couple_bin(m.C, m.S, tw(k), a, pz[i]));
+    v[i] = add(y, add(mul(B1, cm), mul(B2, q)));
+    if (i == 0 && t == 0) {
+      v[0] = add(couple_dc(a, m.cpm.re, T(1) / T(2 * M)), mk<T>(B2.re * m.cpm.re, B2.im * m.cpm.re));
+    }
+    if (i + 1 < Q)
+      cm = mk<T>((cm.re + m.cs.re) + (cm.re * m.cs.re - cm.im * m.cs.im),
+                 (cm.im + m.cs.im) + (cm.re * m.cs.im + cm.im * m.cs.re));
   }
 }
 

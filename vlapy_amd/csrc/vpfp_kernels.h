@@ -29,12 +29,19 @@ constexpr int kMoments = 8;  // n, j, T, q, fv4, vN, f^2, f log f
 VP_HD double trapw(int m, int N) { return (m == 0 || m == N - 1) ? 0.5 : 1.0; }
 
 // ---------------------------------------------------------------------------
-// spectral multiply along a length-2M real sequence held as M complex values
+// spectral multiply along a length-2M real sequence held as M complex values:
+// v in natural order in and out; buf serves the exchanges and ends free
 // ---------------------------------------------------------------------------
 template <class T, int M, int TPT, class Mul, class TW, class Ctx>
 VP_HD void spectral_apply(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, Mul mult, bool act = true) {
   constexpr int Q = M / TPT;
   fft<T, M, TPT, false>(c, v, buf, tw, t, act);
+  // only the partner bins cross threads
+  if (act) {
+#pragma unroll
+    for (int i = 0; i < Q; ++i) buf[pidx(t + i * TPT)] = v[i];
+  }
+  c.sync();
   cx<T> pz[Q];
 #pragma unroll
   for (int i = 0; i < Q; ++i) pz[i] = buf[pidx((M - (t + i * TPT)) & (M - 1))];
@@ -333,9 +340,9 @@ struct RowArgs {
   int field_pro;
   FieldArgs fld;
   // delta-f storage: f holds f - B(v) for a fixed background B (bg [nv],
-  // FP64; unnormalised spectrum bg_hat [nv] in the storage precision); the
-  // kicks shift B spectrally as part of the deviation's multiply (BgPhaseMul),
-  // the collision and moments see B + (f - B) in FP64
+  // FP64; spectrum tables bg_hat [nv] of BgPhaseMul in the storage precision);
+  // the kicks shift B spectrally as part of the deviation's multiply, the
+  // collision and moments see B + (f - B) in FP64
   const double* bg;
   const cx<T>* bg_hat;
 };
@@ -428,14 +435,10 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
     }
   }
   if (chunk) {
-    // natural order -> contiguous chunk of L samples per thread; after a
-    // kick buf already holds the row in natural order (the inverse
-    // transform's last pass ends by reading v from it)
-    if (!(a.flags & RK_KICK_A)) {
+    // natural order -> contiguous chunk of L samples per thread
 #pragma unroll
-      for (int i = 0; i < Q; ++i) buf[pidx(t + i * TPT)] = v[i];
-      c.sync();
-    }
+    for (int i = 0; i < Q; ++i) buf[pidx(t + i * TPT)] = v[i];
+    c.sync();
     double d[L];
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
@@ -603,15 +606,19 @@ VP_HD void field_body(Ctx& c, unsigned char* lds, const FieldArgs& a) {
   mul.okx = okx;
   mul.M = M;
   spectral_apply<double, M, TPT>(c, v, buf, tw, t, mul, act);
-  double acc[2] = {0.0, 0.0};
+  // the TPT threads of the transform hold 2 Q values each: through LDS to one
+  // value per thread, so that the stores are one pass over all FT threads
   if (act) {
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
       const int j = t + i * TPT;
-      field_finish<FT>(c, a, 2 * j, v[i].re, rs, acc);
-      field_finish<FT>(c, a, 2 * j + 1, v[i].im, rs, acc);
+      rho[2 * j] = v[i].re;
+      rho[2 * j + 1] = v[i].im;
     }
   }
+  c.sync();
+  double acc[2] = {0.0, 0.0};
+  for (int x = c.tid; x < Cfg::nx; x += FT) field_finish<FT>(c, a, x, rho[x], rs, acc);
   if (a.series) {
     row_sum<FT, 2>(c, acc, rs);
     if (c.tid == 0) {
@@ -754,13 +761,13 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
     vcol = a.v[tile * C + cc];
   };
   if (t0 < t1) load(t0, nxt, vc_next);
+  c.sync();  // twiddle tables staged
   for (int tile = t0; tile < t1; ++tile) {
     const int col = tile * C + cc;
 #pragma unroll
     for (int i = 0; i < Q; ++i) v[i] = nxt[i];
     const double vc = vc_next;
     if (tile + 1 < t1) load(tile + 1, nxt, vc_next);
-    c.sync();  // twiddle tables staged (first tile) / buffer free (later tiles)
     spectral_apply<T, M, TPT>(c, v, buf, tw, t, PhaseMul<T>((dk * a.dt) * vc, M, t, TPT));
     T* fo = a.f_out + foff + col;
     const double w = trapw(col, a.nv);
