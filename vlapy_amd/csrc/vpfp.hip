@@ -143,15 +143,26 @@ __global__ __launch_bounds__((vp::RowCfg<T, M, Q>::wg)) void k_tri(vp::TriArgs<T
   vp::tri_body<T, M, Q>(c, lds, a);
 }
 
-// Twiddles exp(-2 pi i n / N) built on the device (vpfp_field_noalloc):
-// split = 0: the full table w[n], n < N; split = 1: [lo | hi] with
-// lo[j] = W_N^j (j < 64), hi[h] = W_N^{64 h} (h < N / 64), the layout of
-// split_twiddles for N > vp::kTwFull
+// Twiddles built on the device (vpfp_field_noalloc).  split = 0: the full
+// table w[n] = exp(-2 pi i n / N), n < N; split = 1 (N a power of two >= 4):
+// the field kernel's tables (vp::Tw), W_N^k for k < M = N/2, then the passes of
+// radix 8 after NS = 8, 64, ... points (the last pass's radix is what is left),
+// less than N entries in all
 __global__ __launch_bounds__(256) void k_twiddles(cx<double>* w, int N, int split) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n_entries = split ? 64 + (N / 64 > 1 ? N / 64 : 1) : N;
-  if (i >= n_entries) return;
-  const int n = split ? (i < 64 ? i : 64 * (i - 64)) : i;
+  const int M = N / 2;
+  long long n = i;  // the entry is exp(-2 pi i n / N)
+  if (split && i >= M) {
+    const int e = i - M;
+    if (M <= 8 || e >= M - 8) return;
+    int NS = 8;
+    while (e >= NS * 8 - 8) NS *= 8;
+    const int R = M / NS < 8 ? M / NS : 8;
+    const int r = (e - (NS - 8)) / NS + 1, k = (e - (NS - 8)) % NS;
+    n = (long long)(N / (NS * R)) * r * k;
+  } else if (i >= N) {
+    return;
+  }
   double sn, cs;
   sincospi(2.0 * (double)n / (double)N, &sn, &cs);
   w[i] = vp::mk<double>(cs, -sn);
@@ -369,9 +380,9 @@ struct vpfp_plan_s {
   double* bg = nullptr;          // M(v_m) [nv] (FP64) and its spectrum tables [nv] (storage precision)
   void* bg_hat = nullptr;
   double *kx = nullptr, *okx = nullptr, *v = nullptr, *kv = nullptr;
-  void* tw_v = nullptr;          // cx<T> [lo | hi] tables for nv
-  void* tw_x = nullptr;          // cx<T> [lo | hi] tables for nx
-  cx<double>* tw_xs = nullptr;   // cx<double> [lo | hi] tables for nx (field)
+  void* tw_v = nullptr;          // cx<T> twiddle tables for nv (vp::Tw)
+  void* tw_x = nullptr;          // cx<T> twiddle tables for nx
+  cx<double>* tw_xs = nullptr;   // cx<double> twiddle tables for nx (field)
   cx<double>* tw_xd = nullptr;   // cx<double>[nx] full table (direct-DFT field)
   void* fcopy = nullptr;         // [nx][nv] storage type: f after a step (vpfp_step_n_store's x-modes)
   double* dens = nullptr;        // [max(ntiles,1)][nx]
@@ -416,18 +427,42 @@ std::vector<cx<T>> twiddles(int N) {
   return w;
 }
 
-// Twiddle tables as the kernels stage them: the full W_N^i (i < N) when
-// N <= vp::kTwFull, else [lo | hi]: lo[j] = W_N^j (j < 64), hi[h] = W_N^{64 h}
+// Twiddle tables vp::Tw of an N-point real transform (N a power of two >= 4;
+// other sizes have none): W_N^k for k < M = N/2, then for each Q of `qs` the
+// passes of a transform with Q values per thread, M entries each.  The values
+// come from one octant of long double cosines and sines.
 template <class T>
-std::vector<cx<T>> split_twiddles(int N) {
-  if (vp::tw_full(N, (int)sizeof(cx<T>))) return twiddles<T>(N);
-  const int nhi = N / 64 > 1 ? N / 64 : 1;
-  std::vector<cx<T>> w(64 + nhi);
+std::vector<cx<T>> fft_tables(int N, std::initializer_list<int> qs) {
+  const int M = N / 2;
+  if (N < 4 || (N & (N - 1))) return std::vector<cx<T>>(1);
   const long double two_pi = 6.283185307179586476925286766559L;
-  for (int j = 0; j < 64 + nhi; ++j) {
-    const long double n = j < 64 ? (long double)j : (long double)(64 * (j - 64));
-    const long double a = two_pi * n / (long double)N;
-    w[j] = vp::mk<T>((T)(double)cosl(a), (T)(double)(-sinl(a)));
+  std::vector<cx<T>> full(N);
+  auto set = [&](int n, long double c, long double s) {  // exp(-2 pi i n / N) = (c, -s)
+    full[n & (N - 1)] = vp::mk<T>((T)(double)c, (T)(double)(-s));
+  };
+  for (int n = 0; 8 * n <= N; ++n) {
+    const long double a = two_pi * (long double)n / (long double)N;
+    const long double c = cosl(a), s = 8 * n == N ? c : sinl(a);
+    const int q = N / 4;
+    for (int h = 0; h < 2; ++h) {
+      set(2 * h * q + n, h ? -c : c, h ? -s : s);
+      set(2 * h * q + q - n, h ? -s : s, h ? -c : c);
+      set((2 * h + 1) * q + n, h ? s : -s, h ? -c : c);
+      set((2 * h + 2) * q - n, h ? c : -c, h ? -s : s);
+    }
+  }
+  std::vector<cx<T>> w(M * (1 + qs.size()));
+  std::copy(full.begin(), full.begin() + M, w.begin());
+  size_t base = M;
+  for (int Q : qs) {
+    const int R0 = M < Q ? M : Q;
+    for (int NS = R0; NS < M;) {
+      const int R = M / NS < Q ? M / NS : Q;
+      for (int r = 1; r < R; ++r)
+        for (int k = 0; k < NS; ++k) w[base + NS - R0 + (size_t)(r - 1) * NS + k] = full[(size_t)(N / (NS * R)) * r * k];
+      NS *= R;
+    }
+    base += M;
   }
   return w;
 }
@@ -470,9 +505,9 @@ template <class T>
 int make_tables(vpfp_plan_s* p) {
   cx<T>* dv_ = nullptr;
   cx<T>* dx_ = nullptr;
-  if (int rc = put(p, &dv_, split_twiddles<T>(p->nv))) return rc;
-  if (int rc = put(p, &dx_, split_twiddles<T>(p->nx))) return rc;
-  if (int rc = put(p, &p->tw_xs, split_twiddles<double>(p->nx))) return rc;
+  if (int rc = put(p, &dv_, fft_tables<T>(p->nv, {8, 4, 16}))) return rc;
+  if (int rc = put(p, &dx_, fft_tables<T>(p->nx, {8, 4, 16}))) return rc;
+  if (int rc = put(p, &p->tw_xs, fft_tables<double>(p->nx, {8}))) return rc;
   if (int rc = put(p, &p->tw_xd, twiddles<double>(p->nx))) return rc;
   p->tw_v = dv_;
   p->tw_x = dx_;
@@ -904,9 +939,9 @@ template <class T>
 int batch_tables(vpfp_batch_s* b) {
   cx<T>* tv = nullptr;
   cx<T>* tx = nullptr;
-  if (int rc = bput(b, &tv, split_twiddles<T>(b->nv))) return rc;
-  if (int rc = bput(b, &tx, split_twiddles<T>(b->nx))) return rc;
-  if (int rc = bput(b, &b->tw_xs, split_twiddles<double>(b->nx))) return rc;
+  if (int rc = bput(b, &tv, fft_tables<T>(b->nv, {8, 4, 16}))) return rc;
+  if (int rc = bput(b, &tx, fft_tables<T>(b->nx, {8, 4, 16}))) return rc;
+  if (int rc = bput(b, &b->tw_xs, fft_tables<double>(b->nx, {8}))) return rc;
   b->tw_v = tv;
   b->tw_x = tx;
   return VPFP_OK;
@@ -1763,11 +1798,10 @@ int vpfp_field_noalloc(int nx, int nv, int precision, double dv, const double* o
   double* dens = reinterpret_cast<double*>(base);
   cx<double>* tw = reinterpret_cast<cx<double>*>(base + kNoAllocTwOffset);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // power-of-two nx: the FFT field kernel in one workgroup (tables as
-  // split_twiddles lays them out); any other nx: the direct DFT (full table)
+  // power-of-two nx: the FFT field kernel in one workgroup (its pass tables);
+  // any other nx: the direct DFT (full table)
   const bool pow2 = is_pow2(nx) && nx >= 4;
-  const int split = (pow2 && !vp::tw_full(nx, (int)sizeof(cx<double>))) ? 1 : 0;
-  const int entries = split ? 64 + (nx / 64 > 1 ? nx / 64 : 1) : nx;
+  const int split = pow2 ? 1 : 0, entries = nx;
   hipLaunchKernelGGL(k_twiddles, dim3((entries + 255) / 256), dim3(256), 0, s, tw, nx, split);
   if (int rc = launched()) return rc;
   // n(x) = dv * trapz row sums: every entry is written before it is read

@@ -319,46 +319,29 @@ VP_HD void dft(cx<T>* x) {
 }
 
 // ---------------------------------------------------------------------------
-// Twiddles W_N^i = exp(-2 pi i i / N) staged in LDS.  Large N: two small
-// tables, W_N^i = hi[i >> 6] * lo[i & 63], hi[h] = W_N^{64 h}, lo[j] = W_N^j,
-// global layout [lo: 64 entries | hi: max(1, N/64) entries].
+// Twiddle tables of an N = 2M point real transform, in global memory:
+//   [ W_N^k, k < M | passes for Q = 8 | passes for Q = 4 | passes for Q = 16 ],
+// M entries each (the field's table ends after the second).  A pass of radix R
+// after NS = R0 R1 ... points (R0 the first radix) reads W_{NS R}^{r k} from
+// entry NS - R0 + (r - 1) NS + k of its Q's part, so that the lanes of a wave
+// read consecutive entries.  They come through L1 while the passes exchange
+// through LDS; each is loaded before the barrier ahead of its use.  Staged in
+// LDS instead, the table limited the workgroups on a CU (16 KiB of 25 for an
+// FP64 row of nv = 1024) and its strided reads conflicted on the banks: scan
+// step of 512 FP64 instances 669 -> 594 us, 1024 x 8192 FP64 218 -> 195.
 // ---------------------------------------------------------------------------
-// For N <= kTwFull the whole table W_N^i, i < N, is staged instead: one LDS
-// read per twiddle and no complex product.  Larger full tables cost more than
-// they save: every workgroup stages its table from L2, and a full FP32 table
-// for N = 2048 (16 KiB per one-row workgroup) doubled the row kernel's L2
-// reads and measured 6 % slower at nv = 2048 than the two-level one.
-constexpr int kTwFull = 1024;
-VP_HD constexpr bool tw_full(int N, int bytes) { return bytes > 0 && N <= kTwFull; }
-VP_HD constexpr int tw_entries(int N, int bytes) {
-  return tw_full(N, bytes) ? N : 64 + (N / 64 > 1 ? N / 64 : 1);
-}
+VP_HD constexpr int tw_slot(int Q) { return Q == 4 ? 2 : Q == 16 ? 3 : 1; }
 
-// B: bytes of one complex entry (sizeof(cx<T>))
-template <int N, int B>
-struct TwSize {
-  static constexpr bool full = tw_full(N, B);
-  static constexpr int total = tw_entries(N, B);
-};
-
-template <class T, bool FULL = false>
+template <class T>
 struct Tw {
-  const cx<T>* t;  // LDS copy: W_N^i (FULL) or [lo | hi]
-  VP_HD cx<T> operator()(int i) const {
-    if constexpr (FULL) {
-      return t[i];
-    } else {
-      const cx<T> lo = t[i & 63];
-      if (i < 64) return lo;
-      return mul(t[64 + (i >> 6)], lo);
-    }
-  }
+  const cx<T>* w;  // W_N^k
+  const cx<T>* p;  // pass tables of the transform's Q
 };
 
-// all threads copy the table to LDS (no barrier here)
-template <class T, int N, class Ctx>
-VP_HD void tw_stage(Ctx& c, cx<T>* dst, const cx<T>* src) {
-  for (int i = c.tid; i < TwSize<N, (int)sizeof(cx<T>)>::total; i += c.nthr) dst[i] = src[i];
+// the tables at `tab` for Q values per thread (Q = M < 8: one pass, no table)
+template <int M, int Q, class T>
+VP_HD Tw<T> tw_at(const cx<T>* tab) {
+  return Tw<T>{tab, tab + M * (Q == M ? 0 : tw_slot(Q))};
 }
 
 // ---------------------------------------------------------------------------
@@ -373,17 +356,38 @@ VP_HD void tw_stage(Ctx& c, cx<T>* dst, const cx<T>* src) {
 // already has.  Only the passes before the last go through `buf`; the
 // transform ends with the data in natural order in v and `buf` free.
 //
-// tw(n) = exp(-2 pi i n / (2M)); the M-point twiddle W_M^n is tw(2n).
 // ---------------------------------------------------------------------------
-// `act` false: the thread only takes part in the barriers (no LDS writes).
-template <class T, int M, int TPT, bool INV, int NS = 1, class TW, class Ctx>
-VP_HD void fft(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, bool act = true) {
-  constexpr int Q = M / TPT;
+template <int M, int TPT, int NS>
+struct Pass {
+  static constexpr int Q = M / TPT;
   static_assert(Q >= 2 && Q * TPT == M, "each thread must hold at least two values");
-  constexpr int RMAX = Q < 16 ? Q : 16;
-  constexpr int R = (M / NS) < RMAX ? (M / NS) : RMAX;
-  constexpr int NB = Q / R;
+  static constexpr int RMAX = Q < 16 ? Q : 16;
+  static constexpr int R0 = M < RMAX ? M : RMAX;
+  static constexpr int R = (M / NS) < RMAX ? (M / NS) : RMAX;
+  static constexpr int NB = Q / R;
   static_assert(NB * R == Q, "radix must divide the per-thread count");
+  // j mod NS is the same for all of a thread's butterflies when NS divides TPT
+  static constexpr int NK = NS > TPT ? NB : 1;
+  static constexpr int NW = NK * (R - 1) > 0 ? NK * (R - 1) : 1;
+};
+
+template <class T, int M, int TPT, int NS>
+VP_HD void load_twiddles(cx<T>* w, const Tw<T>& tw, int t) {
+  using P = Pass<M, TPT, NS>;
+#pragma unroll
+  for (int q = 0; q < P::NK; ++q) {
+    const cx<T>* p = tw.p + (NS - P::R0) + ((t + q * TPT) & (NS - 1));
+#pragma unroll
+    for (int r = 1; r < P::R; ++r) w[q * (P::R - 1) + r - 1] = p[(r - 1) * NS];
+  }
+}
+
+// passes from NS on; w: this pass's twiddles (NS > 1).  `act` false: the
+// thread only takes part in the barriers (no LDS writes).
+template <class T, int M, int TPT, bool INV, int NS, class Ctx>
+VP_HD void fft_passes(Ctx& c, cx<T>* v, cx<T>* buf, const Tw<T>& tw, int t, bool act, const cx<T>* w) {
+  using P = Pass<M, TPT, NS>;
+  constexpr int Q = P::Q, R = P::R, NB = P::NB;
 #pragma unroll
   for (int q = 0; q < NB; ++q) {
     const int j = t + q * TPT;
@@ -392,11 +396,9 @@ VP_HD void fft(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, bool act = tru
 #pragma unroll
     for (int r = 0; r < R; ++r) u[r] = v[q + r * NB];
     if constexpr (NS > 1) {
+      const cx<T>* wq = w + (P::NK > 1 ? q * (R - 1) : 0);
 #pragma unroll
-      for (int r = 1; r < R; ++r) {
-        const cx<T> w = tw(2 * (r * k * (M / (NS * R))));
-        u[r] = INV ? mulc(u[r], w) : mul(u[r], w);
-      }
+      for (int r = 1; r < R; ++r) u[r] = INV ? mulc(u[r], wq[r - 1]) : mul(u[r], wq[r - 1]);
     }
     dft<R, INV>(u);
     if constexpr (NS * R < M) {
@@ -411,12 +413,19 @@ VP_HD void fft(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, bool act = tru
     }
   }
   if constexpr (NS * R < M) {
+    cx<T> wn[Pass<M, TPT, NS * R>::NW];
+    load_twiddles<T, M, TPT, NS * R>(wn, tw, t);
     c.sync();
 #pragma unroll
     for (int i = 0; i < Q; ++i) v[i] = buf[pidx(t + i * TPT)];
     c.sync();
-    fft<T, M, TPT, INV, NS * R>(c, v, buf, tw, t, act);
+    fft_passes<T, M, TPT, INV, NS * R>(c, v, buf, tw, t, act, wn);
   }
+}
+
+template <class T, int M, int TPT, bool INV, class Ctx>
+VP_HD void fft(Ctx& c, cx<T>* v, cx<T>* buf, const Tw<T>& tw, int t, bool act = true) {
+  fft_passes<T, M, TPT, INV, 1>(c, v, buf, tw, t, act, static_cast<const cx<T>*>(nullptr));
 }
 
 // ---------------------------------------------------------------------------
@@ -538,9 +547,9 @@ struct PoissonMul {
 // F_{k+M} = E_k - W O_k.  After F'_k = P_k F_k, F'_{k+M} = conj(P_{M-k}) F_{k+M}
 // the repacked spectrum Z'_k = (F'_k + F'_{k+M} + i (F'_k - F'_{k+M}) conj W)/N
 // inverse-transforms (unnormalised M-point) to f'_{2j} + i f'_{2j+1}.
-// v[i] holds Z_k and pz[i] holds Z_{M-k} for k = t + i*TPT; tw(k) = W^k.
-template <class T, int M, int TPT, class TW>
-VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, PoissonMul<T>& mult) {
+// v[i] holds Z_k, pz[i] Z_{M-k} and wk[i] W^k for k = t + i*TPT.
+template <class T, int M, int TPT>
+VP_HD void couple(cx<T>* v, const cx<T>* pz, const cx<T>* wk, int t, PoissonMul<T>& mult) {
   constexpr int Q = M / TPT;
   const T invN = T(1) / T(2 * M);
   const T h = T(0.5);
@@ -550,7 +559,7 @@ VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, PoissonMul<T>&
     const cx<T> a = v[i], p = pz[i];
     const cx<T> E = mk<T>((a.re + p.re) * h, (a.im - p.im) * h);
     const cx<T> O = mk<T>((a.im + p.im) * h, (p.re - a.re) * h);
-    const cx<T> W = tw(k);
+    const cx<T> W = wk[i];
     const cx<T> WO = mul(W, O);
     const cx<T> Fk = add(E, WO), Fkm = sub(E, WO);
     cx<T> pk, pmk;
@@ -578,21 +587,21 @@ VP_HD cx<T> couple_dc(cx<T> a, T nyq, T invN) {
   return mk<T>((f0 + g2) * invN, (f0 - g2) * invN);
 }
 
-template <class T, int M, int TPT, class TW>
-VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, PhaseMul<T>& m) {
+template <class T, int M, int TPT>
+VP_HD void couple(cx<T>* v, const cx<T>* pz, const cx<T>* wk, int t, PhaseMul<T>& m) {
   constexpr int Q = M / TPT;
   cx<T> cur = m.cur;
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
     const cx<T> a = v[i];
-    v[i] = mul(cur, couple_bin(m.C, m.S, tw(t + i * TPT), a, pz[i]));
+    v[i] = mul(cur, couple_bin(m.C, m.S, wk[i], a, pz[i]));
     if (i == 0 && t == 0) v[0] = couple_dc(a, T(-2) * m.S * m.S, T(1) / T(2 * M));
     if (i + 1 < Q) cur = mul(cur, m.step);
   }
 }
 
-template <class T, int M, int TPT, class TW>
-VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, BgPhaseMul<T>& m) {
+template <class T, int M, int TPT>
+VP_HD void couple(cx<T>* v, const cx<T>* pz, const cx<T>* wk, int t, BgPhaseMul<T>& m) {
   constexpr int Q = M / TPT;
   const cx<T> kap = half_phase(m.C, m.S, T(1) / T(M));
   cx<T> cm = m.cm;
@@ -604,7 +613,7 @@ VP_HD void couple(cx<T>* v, const cx<T>* pz, const TW& tw, int t, BgPhaseMul<T>&
     const cx<T> pk = mk<T>(kap.re + (kap.re * cm.re - kap.im * cm.im), kap.im + (kap.re * cm.im + kap.im * cm.re));
     const cx<T> q = mk<T>((m.cpm.re + cm.re) + (m.cpm.re * cm.re - m.cpm.im * cm.im),
                           (m.cpm.im + cm.im) + (m.cpm.re * cm.im + m.cpm.im * cm.re));
-    const cx<T> y = mul(pk, couple_bin(m.C, m.S, tw(k), a, pz[i]));
+    const cx<T> y = mul(pk, couple_bin(m.C, m.S, wk[i], a, pz[i]));
     v[i] = add(y, add(mul(B1, cm), mul(B2, q)));
     if (i == 0 && t == 0) {
       v[0] = add(couple_dc(a, m.cpm.re, T(1) / T(2 * M)), mk<T>(B2.re * m.cpm.re, B2.im * m.cpm.re));

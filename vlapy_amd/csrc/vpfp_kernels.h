@@ -32,8 +32,8 @@ VP_HD double trapw(int m, int N) { return (m == 0 || m == N - 1) ? 0.5 : 1.0; }
 // spectral multiply along a length-2M real sequence held as M complex values:
 // v in natural order in and out; buf serves the exchanges and ends free
 // ---------------------------------------------------------------------------
-template <class T, int M, int TPT, class Mul, class TW, class Ctx>
-VP_HD void spectral_apply(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, Mul mult, bool act = true) {
+template <class T, int M, int TPT, class Mul, class Ctx>
+VP_HD void spectral_apply(Ctx& c, cx<T>* v, cx<T>* buf, const Tw<T>& tw, int t, Mul mult, bool act = true) {
   constexpr int Q = M / TPT;
   fft<T, M, TPT, false>(c, v, buf, tw, t, act);
   // only the partner bins cross threads
@@ -41,12 +41,15 @@ VP_HD void spectral_apply(Ctx& c, cx<T>* v, cx<T>* buf, const TW& tw, int t, Mul
 #pragma unroll
     for (int i = 0; i < Q; ++i) buf[pidx(t + i * TPT)] = v[i];
   }
+  cx<T> wk[Q];
+#pragma unroll
+  for (int i = 0; i < Q; ++i) wk[i] = tw.w[t + i * TPT];
   c.sync();
   cx<T> pz[Q];
 #pragma unroll
   for (int i = 0; i < Q; ++i) pz[i] = buf[pidx((M - (t + i * TPT)) & (M - 1))];
   c.sync();
-  couple<T, M, TPT>(v, pz, tw, t, mult);
+  couple<T, M, TPT>(v, pz, wk, t, mult);
   fft<T, M, TPT, true>(c, v, buf, tw, t, act);
 }
 
@@ -157,7 +160,7 @@ struct FieldArgs {
   double* rho_g;          // [nx] global scratch when the grid has several workgroups
   unsigned int* counter;  // arrival counter (zero between launches)
   const double* okx;      // [nx]
-  const cx<double>* tw;   // pow2 kernel: twiddle tables [lo | hi]; DFT kernel: exp(-2 pi i n / nx), n < nx
+  const cx<double>* tw;   // pow2 kernel: twiddle tables of nx (Tw); DFT kernel: exp(-2 pi i n / nx), n < nx
   const double* driver;   // [nx] or null
   double* e_out;          // [nx]
   double* e_out2;         // [nx] or null
@@ -327,7 +330,7 @@ struct RowArgs {
   double dk;         // kv[1] of the fftfreq table
   double v0, dvv;    // v_m = v0 + m dvv
   double dv;
-  const cx<T>* tw;   // twiddle tables of exp(-2 pi i n / nv), [lo | hi]
+  const cx<T>* tw;   // twiddle tables of nv (Tw)
   double nu_dt;
   int op_dg;
   double* moments;  // [kMoments][nx]
@@ -351,17 +354,16 @@ template <class T, int M, int Q>
 struct RowCfg {
   static constexpr int TPT = M / Q;
   static constexpr int L = 2 * Q;
-  static constexpr int tw_bytes = (TwSize<2 * M, (int)sizeof(cx<T>)>::total * (int)sizeof(cx<T>) + 15) & ~15;
   static constexpr int fft_bytes = Padded<M>::size * (int)sizeof(cx<T>);
   static constexpr int red_bytes = 8 * TPT * 8;
   static constexpr int region = ((fft_bytes > red_bytes ? fft_bytes : red_bytes) + 15) & ~15;
   static constexpr int wg = TPT >= 64 ? TPT : 64;
   static constexpr int rows = wg / TPT;
   static constexpr int sum_bytes = (TPT > 64 ? TPT / 64 : 1) * kMoments * 8;
-  // the field prologue (field_rows) runs before the twiddles and row buffers
-  // are staged and overlays them from offset 0
+  // the field prologue (field_rows) runs before the row buffers are used and
+  // overlays them from offset 0
   static constexpr int pro_bytes = ProCfg<wg>::bytes;
-  static constexpr int main_bytes = tw_bytes + rows * region + sum_bytes;
+  static constexpr int main_bytes = rows * region + sum_bytes;
   static constexpr int lds = main_bytes > pro_bytes ? main_bytes : pro_bytes;
   // minimum waves per SIMD asked of the register allocator: 3 (168 VGPRs,
   // small spills) measured faster than 2 for FP32 rows with M <= 1024 (the
@@ -381,11 +383,9 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
   const int row = c.bid * Cfg::rows + rl;
   const bool valid = row < a.nx;
   const int rowc = valid ? row : a.nx - 1;
-  cx<T>* twl = reinterpret_cast<cx<T>*>(lds);
-  unsigned char* base = lds + Cfg::tw_bytes;
-  cx<T>* buf = reinterpret_cast<cx<T>*>(base + rl * Cfg::region);
-  double* red = reinterpret_cast<double*>(base + rl * Cfg::region);
-  double* rs = reinterpret_cast<double*>(base + Cfg::rows * Cfg::region);
+  cx<T>* buf = reinterpret_cast<cx<T>*>(lds + rl * Cfg::region);
+  double* red = reinterpret_cast<double*>(lds + rl * Cfg::region);
+  double* rs = reinterpret_cast<double*>(lds + Cfg::rows * Cfg::region);
 
   const cx<T>* src = reinterpret_cast<const cx<T>*>(a.f_in + (size_t)rowc * a.nv);
   cx<T> v[Q];
@@ -397,13 +397,11 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
     const int nr = a.nx - row0 < Cfg::rows ? a.nx - row0 : Cfg::rows;
     field_rows<Cfg::wg>(c, a.fld, lds, row0, nr);
     e = reinterpret_cast<const double*>(lds + ProCfg<Cfg::wg>::erow_off)[valid ? row : 0];
-    c.sync();  // every thread has its E before the twiddles overwrite the prologue's LDS
+    c.sync();  // every thread has its E before the transforms overwrite the prologue's LDS
   } else if (a.flags & (RK_KICK_A | RK_KICK_B)) {
     e = a.e[rowc];
   }
-  tw_stage<T, 2 * M>(c, twl, a.tw);
-  c.sync();
-  const Tw<T, TwSize<2 * M, (int)sizeof(cx<T>)>::full> tw{twl};
+  const Tw<T> tw = tw_at<M, Q>(a.tw);
 
   // kick by shift a: f(v) -> f(v - a), spectrally (the background's shift too
   // under delta-f storage)
@@ -564,10 +562,9 @@ struct FieldCfg {
   static constexpr int TPT = M / Q;
   static constexpr int nx = 2 * M;
   static constexpr int tmp_n = (nx > FT ? nx : FT);
-  static constexpr int tw_bytes = TwSize<nx, 16>::total * 16;
   static constexpr int work = (Padded<M>::size * 16 > tmp_n * 8) ? Padded<M>::size * 16 : tmp_n * 8;
-  // [twiddles | okx (nx) | rho (nx) | fft buffer / reduction scratch | row_sum scratch | flag]
-  static constexpr int lds = tw_bytes + 2 * nx * 8 + work + 64 + 16;
+  // [okx (nx) | rho (nx) | fft buffer / reduction scratch | row_sum scratch | flag]
+  static constexpr int lds = 2 * nx * 8 + work + 64 + 16;
 };
 
 // TAIL: called by the last workgroup of the drift kernel, which reads every
@@ -577,8 +574,7 @@ VP_HD void field_body(Ctx& c, unsigned char* lds, const FieldArgs& a) {
   using Cfg = FieldCfg<M, Q, FT>;
   constexpr int TPT = Cfg::TPT;
   static_assert(TPT <= FT, "field transform needs at most FT threads");
-  cx<double>* twl = reinterpret_cast<cx<double>*>(lds);
-  double* okx = reinterpret_cast<double*>(lds + Cfg::tw_bytes);
+  double* okx = reinterpret_cast<double*>(lds);
   double* rho = okx + Cfg::nx;
   cx<double>* buf = reinterpret_cast<cx<double>*>(rho + Cfg::nx);
   double* tmp = reinterpret_cast<double*>(buf);
@@ -590,10 +586,10 @@ VP_HD void field_body(Ctx& c, unsigned char* lds, const FieldArgs& a) {
   } else {
     if (!field_gather<FT>(c, a, rho, tmp, flag)) return;
   }
-  tw_stage<double, Cfg::nx>(c, twl, a.tw);
   for (int x = c.tid; x < Cfg::nx; x += FT) okx[x] = a.okx[x];
   c.sync();
-  const Tw<double, TwSize<Cfg::nx, 16>::full> tw{twl};
+  static_assert(Q == M || Q == 8 || M > 2048, "the field (nx <= 4096) has the pass tables of Q = 8");
+  const Tw<double> tw = tw_at<M, Q>(a.tw);
   const bool act = c.tid < TPT;
   const int t = act ? c.tid : 0;
   cx<double> v[Q];
@@ -679,7 +675,7 @@ struct DriftArgs {
   double dt;
   double dk;         // kx[1] of the fftfreq table
   const double* v;   // [nv]
-  const cx<T>* tw;   // twiddle tables of exp(-2 pi i n / nx), [lo | hi]
+  const cx<T>* tw;   // twiddle tables of nx (Tw)
   double* dens;      // [gridDim][nx] partial sums (unscaled), or null
   int fuse_field;    // 1: the last workgroup to finish solves the field (fld)
   FieldArgs fld;     // field arguments for the fused tail (part = dens)
@@ -713,8 +709,7 @@ struct DriftCfg {
   // on different LDS banks (an even multiple of 64 banks made the columns a
   // wave touches collide)
   static constexpr int stride = Padded<M>::size | 1;
-  static constexpr int tw_bytes = (TwSize<2 * M, (int)sizeof(cx<T>)>::total * (int)sizeof(cx<T>) + 15) & ~15;
-  static constexpr int own = tw_bytes + C * stride * (int)sizeof(cx<T>);
+  static constexpr int own = C * stride * (int)sizeof(cx<T>);
   // fused field tail (small grids): M-point Poisson transform on the same workgroup
   static constexpr int fq = M < 8 ? M : 8;
   static constexpr bool tail = M <= 128 && (M / fq) <= wg;
@@ -728,14 +723,12 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
   constexpr int TPT = Cfg::TPT;
   const int cc = c.tid % C;
   const int t = c.tid / C;
-  cx<T>* twl = reinterpret_cast<cx<T>*>(lds);
-  cx<T>* buf = reinterpret_cast<cx<T>*>(lds + Cfg::tw_bytes) + cc * Cfg::stride;
+  cx<T>* buf = reinterpret_cast<cx<T>*>(lds) + cc * Cfg::stride;
   const size_t nv = (size_t)a.nv;
   const int inst = c.bidy;
   const size_t foff = (size_t)inst * (size_t)a.nx * nv;
   const double dk = a.dk_inst ? a.dk_inst[inst] : a.dk;
-  tw_stage<T, 2 * M>(c, twl, a.tw);
-  const Tw<T, TwSize<2 * M, (int)sizeof(cx<T>)>::full> tw{twl};
+  const Tw<T> tw = tw_at<M, Q>(a.tw);
   double acc[2 * Q];
 #pragma unroll
   for (int i = 0; i < 2 * Q; ++i) acc[i] = 0.0;
@@ -761,7 +754,6 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
     vcol = a.v[tile * C + cc];
   };
   if (t0 < t1) load(t0, nxt, vc_next);
-  c.sync();  // twiddle tables staged
   for (int tile = t0; tile < t1; ++tile) {
     const int col = tile * C + cc;
 #pragma unroll
