@@ -405,11 +405,11 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
 
   // kick by shift a: f(v) -> f(v - a), spectrally (the background's shift too
   // under delta-f storage)
-  auto kick = [&](double shift) {
+  auto phases = [&](double shift) {
     if constexpr (BG)
-      spectral_apply<T, M, TPT>(c, v, buf, tw, t, BgPhaseMul<T>(a.dk * shift, M, t, TPT, a.bg_hat));
+      return BgPhaseMul<T>(a.dk * shift, M, t, TPT, a.bg_hat);
     else
-      spectral_apply<T, M, TPT>(c, v, buf, tw, t, PhaseMul<T>(a.dk * shift, M, t, TPT));
+      return PhaseMul<T>(a.dk * shift, M, t, TPT);
   };
   const bool chunk = (a.flags & (RK_COLLIDE | RK_MOMENTS)) != 0;
   // two half kicks by the same field with nothing between them (no
@@ -417,7 +417,11 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
   // kick by the sum of the shifts: the phase factors multiply exactly, so
   // one transform pair replaces two
   const bool merged = (a.flags & RK_KICK_A) && (a.flags & RK_KICK_B) && !chunk && !a.f_copy;
-  if (a.flags & RK_KICK_A) kick((merged ? a.dt_a + a.dt_b : a.dt_a) * e);
+  decltype(phases(0.0)) ph;
+  if (a.flags & RK_KICK_A) {
+    ph = phases((merged ? a.dt_a + a.dt_b : a.dt_a) * e);
+    spectral_apply<T, M, TPT>(c, v, buf, tw, t, ph);
+  }
 
   if (a.f_copy && !chunk && valid) {
     // copy only: natural order, one complex pair per value (coalesced)
@@ -512,7 +516,12 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
     c.sync();
   }
 
-  if ((a.flags & RK_KICK_B) && !merged) kick(a.dt_b * e);
+  if ((a.flags & RK_KICK_B) && !merged) {
+    // the second half kick of a step shifts by the first's amount: its phases
+    // are kept through the collision
+    if (!(a.flags & RK_KICK_A) || a.dt_b != a.dt_a) ph = phases(a.dt_b * e);
+    spectral_apply<T, M, TPT>(c, v, buf, tw, t, ph);
+  }
 
   if (valid && a.f_out) {
     cx<T>* dst = reinterpret_cast<cx<T>*>(a.f_out + (size_t)row * a.nv);
