@@ -415,35 +415,30 @@ int upload(void* dst, const void* src, size_t bytes) {
   return VPFP_OK;
 }
 
-// exp(-2 pi i n / N) for n < N in long double, rounded
-template <class T>
-std::vector<cx<T>> twiddles(int N) {
-  std::vector<cx<T>> w(N);
-  const long double two_pi = 6.283185307179586476925286766559L;
-  for (int n = 0; n < N; ++n) {
-    const long double a = two_pi * (long double)n / (long double)N;
-    w[n] = vp::mk<T>((T)(double)cosl(a), (T)(double)(-sinl(a)));
+// exp(-2 pi i n / N) for n < N, rounded from long double.  Power-of-two sizes
+// (at most 8192 here) are computed once per process from one octant and kept,
+// 256 KiB in all: evaluated anew, they were 0.1 ms of a plan's creation.
+const std::vector<cx<double>>& unit_circle(int lg) {
+  static std::mutex mu;
+  static std::vector<cx<double>> tab[14];
+  std::lock_guard<std::mutex> lock(mu);
+  std::vector<cx<double>>& w = tab[lg];
+  if (!w.empty()) return w;
+  const int N = 1 << lg;
+  std::vector<cx<double>> full(N);
+  if (N < 4) {
+    for (int n = 0; n < N; ++n) full[n] = vp::mk<double>(n ? -1.0 : 1.0, 0.0);
+    w.swap(full);
+    return w;
   }
-  return w;
-}
-
-// Twiddle tables vp::Tw of an N-point real transform (N a power of two >= 4;
-// other sizes have none): W_N^k for k < M = N/2, then for each Q of `qs` the
-// passes of a transform with Q values per thread, M entries each.  The values
-// come from one octant of long double cosines and sines.
-template <class T>
-std::vector<cx<T>> fft_tables(int N, std::initializer_list<int> qs) {
-  const int M = N / 2;
-  if (N < 4 || (N & (N - 1))) return std::vector<cx<T>>(1);
   const long double two_pi = 6.283185307179586476925286766559L;
-  std::vector<cx<T>> full(N);
-  auto set = [&](int n, long double c, long double s) {  // exp(-2 pi i n / N) = (c, -s)
-    full[n & (N - 1)] = vp::mk<T>((T)(double)c, (T)(double)(-s));
+  auto set = [&](int n, double c, double s) {  // exp(-2 pi i n / N) = (c, -s)
+    full[n & (N - 1)] = vp::mk<double>(c, -s);
   };
+  const int q = N / 4;
   for (int n = 0; 8 * n <= N; ++n) {
     const long double a = two_pi * (long double)n / (long double)N;
-    const long double c = cosl(a), s = 8 * n == N ? c : sinl(a);
-    const int q = N / 4;
+    const double c = (double)cosl(a), s = 8 * n == N ? c : (double)sinl(a);
     for (int h = 0; h < 2; ++h) {
       set(2 * h * q + n, h ? -c : c, h ? -s : s);
       set(2 * h * q + q - n, h ? -s : s, h ? -c : c);
@@ -451,15 +446,47 @@ std::vector<cx<T>> fft_tables(int N, std::initializer_list<int> qs) {
       set((2 * h + 2) * q - n, h ? c : -c, h ? -s : s);
     }
   }
+  w.swap(full);
+  return w;
+}
+
+int log2i(int N) {
+  int lg = 0;
+  while ((1 << lg) < N) ++lg;
+  return lg;
+}
+
+// the full table exp(-2 pi i n / N), n < N, any N
+std::vector<cx<double>> twiddles(int N) {
+  if ((N & (N - 1)) == 0 && N <= 8192) return unit_circle(log2i(N));
+  std::vector<cx<double>> w(N);
+  const long double two_pi = 6.283185307179586476925286766559L;
+  for (int n = 0; n < N; ++n) {
+    const long double a = two_pi * (long double)n / (long double)N;
+    w[n] = vp::mk<double>((double)cosl(a), (double)(-sinl(a)));
+  }
+  return w;
+}
+
+// Twiddle tables vp::Tw of an N-point real transform (N a power of two in
+// [4, 8192]; other sizes have none): W_N^k for k < M = N/2, then for each Q of
+// `qs` the passes of a transform with Q values per thread, M entries each.
+template <class T>
+std::vector<cx<T>> fft_tables(int N, std::initializer_list<int> qs) {
+  const int M = N / 2;
+  if (N < 4 || N > 8192 || (N & (N - 1))) return std::vector<cx<T>>(1);
+  const std::vector<cx<double>>& full = unit_circle(log2i(N));
+  auto at = [&](size_t i) { return vp::mk<T>((T)full[i].re, (T)full[i].im); };
   std::vector<cx<T>> w(M * (1 + qs.size()));
-  std::copy(full.begin(), full.begin() + M, w.begin());
+  for (int k = 0; k < M; ++k) w[k] = at(k);
   size_t base = M;
   for (int Q : qs) {
     const int R0 = M < Q ? M : Q;
     for (int NS = R0; NS < M;) {
       const int R = M / NS < Q ? M / NS : Q;
+      const size_t step = (size_t)(N / (NS * R));
       for (int r = 1; r < R; ++r)
-        for (int k = 0; k < NS; ++k) w[base + NS - R0 + (size_t)(r - 1) * NS + k] = full[(size_t)(N / (NS * R)) * r * k];
+        for (int k = 0; k < NS; ++k) w[base + NS - R0 + (size_t)(r - 1) * NS + k] = at(step * r * k);
       NS *= R;
     }
     base += M;
@@ -475,21 +502,16 @@ std::vector<cx<T>> fft_tables(int N, std::initializer_list<int> qs) {
 // synthesis from those rows.
 std::vector<float> dft_matrices(int N) {
   std::vector<float> m(2 * (size_t)N * N);
-  const long double tp = 6.283185307179586476925286766559L;
-  auto ang = [&](long long k, int x) { return tp * (long double)((k * x) % N) / (long double)N; };
+  const std::vector<cx<double>>& w = unit_circle(log2i(N));
+  auto cs = [&](int k, int x) { return w[(size_t)k * x % N].re; };
+  auto sn = [&](int k, int x) { return -w[(size_t)k * x % N].im; };
   for (int row = 0; row < N; ++row)
-    for (int x = 0; x < N; ++x)
-      m[(size_t)row * N + x] = (float)(row <= N / 2 ? cosl(ang(row, x)) : -sinl(ang(row - N / 2, x)));
+    for (int x = 0; x < N; ++x) m[(size_t)row * N + x] = (float)(row <= N / 2 ? cs(row, x) : -sn(row - N / 2, x));
   float* G = m.data() + (size_t)N * N;
   for (int x = 0; x < N; ++x)
-    for (int col = 0; col < N; ++col) {
-      long double v;
-      if (col <= N / 2)
-        v = ((col == 0 || col == N / 2) ? 1.0L : 2.0L) * cosl(ang(col, x)) / N;
-      else
-        v = -2.0L * sinl(ang(col - N / 2, x)) / N;
-      G[(size_t)x * N + col] = (float)v;
-    }
+    for (int col = 0; col < N; ++col)
+      G[(size_t)x * N + col] = (float)(col <= N / 2 ? ((col == 0 || col == N / 2) ? 1.0 : 2.0) * cs(col, x) / N
+                                                    : -2.0 * sn(col - N / 2, x) / N);
   return m;
 }
 
@@ -506,9 +528,13 @@ int make_tables(vpfp_plan_s* p) {
   cx<T>* dv_ = nullptr;
   cx<T>* dx_ = nullptr;
   if (int rc = put(p, &dv_, fft_tables<T>(p->nv, {8, 4, 16}))) return rc;
-  if (int rc = put(p, &dx_, fft_tables<T>(p->nx, {8, 4, 16}))) return rc;
-  if (int rc = put(p, &p->tw_xs, fft_tables<double>(p->nx, {8}))) return rc;
-  if (int rc = put(p, &p->tw_xd, twiddles<double>(p->nx))) return rc;
+  if (int rc = put(p, &dx_, fft_tables<T>(p->nx, {8, 4}))) return rc;
+  if constexpr (sizeof(T) == 8) {
+    p->tw_xs = dx_;
+  } else {
+    if (int rc = put(p, &p->tw_xs, fft_tables<double>(p->nx, {8}))) return rc;
+  }
+  if (int rc = put(p, &p->tw_xd, twiddles(p->nx))) return rc;
   p->tw_v = dv_;
   p->tw_x = dx_;
   return VPFP_OK;
@@ -955,8 +981,12 @@ int batch_tables(vpfp_batch_s* b) {
   cx<T>* tv = nullptr;
   cx<T>* tx = nullptr;
   if (int rc = bput(b, &tv, fft_tables<T>(b->nv, {8, 4, 16}))) return rc;
-  if (int rc = bput(b, &tx, fft_tables<T>(b->nx, {8, 4, 16}))) return rc;
-  if (int rc = bput(b, &b->tw_xs, fft_tables<double>(b->nx, {8}))) return rc;
+  if (int rc = bput(b, &tx, fft_tables<T>(b->nx, {8, 4}))) return rc;
+  if constexpr (sizeof(T) == 8) {
+    b->tw_xs = tx;
+  } else {
+    if (int rc = bput(b, &b->tw_xs, fft_tables<double>(b->nx, {8}))) return rc;
+  }
   b->tw_v = tv;
   b->tw_x = tx;
   return VPFP_OK;
