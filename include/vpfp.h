@@ -154,9 +154,10 @@ int vpfp_step_n(vpfp_plan_t plan, void* f, double* e, int n_steps, const double*
  *   n_modes > 0:  the first n_modes Fourier modes along x of f, f_store
  *                 [n_steps][n_modes][nv] complex128, equal to vpfp_x_modes:
  *                 the row kernel writes f to plan scratch and extra
- *                 workgroups of the next step's field launch sum it over x
+ *                 workgroups of the next step's row launch sum it over x
  *                 (one more launch after the last step).
- * Three launches per step either way.  Under delta-f storage the store holds
+ * Two launches per step either way (three where the field's densities are
+ * summed first).  Under delta-f storage the store holds
  * f itself. */
 int vpfp_step_n_store(vpfp_plan_t plan, void* f, double* e, int n_steps, const double* driver, double* e_hist,
                       double* moments, double* series, void* f_store, int n_modes, void* stream);
@@ -174,8 +175,8 @@ int vpfp_step_n_store(vpfp_plan_t plan, void* f, double* e, int n_steps, const d
  * zero).  e [nx] is the field the 6th-order scheme's first kick uses and
  * becomes the last E.  e_hist [n_steps][nx] (E after each step), moments
  * [n_steps][VPFP_NMOMENTS][nx], series [n_steps][2] (mean E^2 and mean square
- * of the step's last driver) and f_store/n_modes as vpfp_step_n_store (the
- * x-modes by one launch per step) are optional (NULL / 0). */
+ * of the step's last driver) and f_store/n_modes as vpfp_step_n_store are
+ * optional (NULL / 0). */
 #define VPFP_SCHEME_PEFRL 1
 #define VPFP_SCHEME_SIXTH 2
 #define VPFP_SCHEME_FIELDS 5
@@ -273,11 +274,13 @@ int vpfp_batch_background(vpfp_batch_t batch, void* f, int sign, void* stream);
  *               (16 <= nv/2 <= 2048), 8, or 16 (nv/2 >= 256); 0 = by row
  *               count (4 when the grid has few rows, else 8)
  *   drift_tile  x-advection columns per workgroup: 4, 8, 16 or 32 (0 = keep)
- *   fuse_field  1: the last drift workgroup solves the field (nx <= 256);
- *               2: every row workgroup forms the field at its own rows from
- *               the drift's partial densities (direct DFT, nx <= 128);
- *               0 or -1 (default): separate field launch.  Batches always
- *               use the separate launch and report 0.
+ *   fuse_field  0: the field is a launch of its own; 1: the last drift
+ *               workgroup solves it (nx <= 256); 2: every row workgroup forms
+ *               the field at its own rows from the drift's partial densities
+ *               (nx <= 128); -1 (default): as 2 at any nx, the partial
+ *               densities summed by a launch first when they are many.
+ *               Batches always use the separate launch and report 0, the
+ *               higher-order schemes always the -1 rule.
  *   drift_order 1: consecutive column tiles on the workgroups of one XCD
  *               (workgroup b runs on XCD b % 8); 0: tile = workgroup index
  *   drift_tiles column tiles per drift workgroup (1 = one each; a single

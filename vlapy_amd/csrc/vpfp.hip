@@ -67,19 +67,6 @@ template <int M, int Q>
 __global__ __launch_bounds__(kFT) void k_field(vp::FieldArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   VPFP_CTX;
-  if (a.xm_out) {
-    // the previous step's f store beside the solve: workgroups from
-    // xm_blk0 on take one (mode, v) pair per thread
-    if (c.bid >= a.xm_blk0) {
-      GpuCtx x{c.tid, c.nthr, c.bid - a.xm_blk0, c.nblk - a.xm_blk0, 0};
-      if (a.xm_f32)
-        vp::xmodes_body<float>(x, static_cast<const float*>(a.xm_f), a.nx, a.xm_nv, a.xm_n, a.xm_tw, a.xm_out);
-      else
-        vp::xmodes_body<double>(x, static_cast<const double*>(a.xm_f), a.nx, a.xm_nv, a.xm_n, a.xm_tw, a.xm_out);
-      return;
-    }
-    c.nblk = a.xm_blk0;
-  }
   vp::field_body<M, Q, kFT>(c, lds, vp::field_instance(a, c.bidy));
 }
 
@@ -116,10 +103,56 @@ __global__ __launch_bounds__(256) void k_background(T* f, size_t n, int nv, cons
   f[i] = (T)((double)f[i] + sign * bg[m]);
 }
 
-template <class T>
+template <class T, int W>
 __global__ __launch_bounds__(256) void k_density(const T* f, int nx, int nv, double scale, double* part) {
+  __shared__ double rs[4];
   VPFP_CTX;
-  vp::density_body<T>(c, f, nx, nv, scale, part);
+  vp::density_body<T, W>(c, f, nx, nv, scale, part, rs);
+}
+
+// E(x) by the Green's function (vp::green_body) and its table
+__global__ __launch_bounds__(256) void k_green(vp::FieldArgs a) {
+  VPFP_CTX;
+  vp::green_body(c, a);
+}
+
+__global__ __launch_bounds__(256) void k_green_table(const double* okx, const cx<double>* tw, int nx, double* green) {
+  VPFP_CTX;
+  vp::green_table_body(c, okx, tw, nx, green);
+}
+
+// out[x] = sum of the partial density rows at x, kRhoXS columns per workgroup
+constexpr int kRhoXS = 16;
+__global__ __launch_bounds__(kFT) void k_rho(const double* part, int ntiles, int nx, double* out) {
+  __shared__ double tmp[kFT];
+  const int XS = nx < kRhoXS ? nx : kRhoXS, G = kFT / XS;
+  const int xl = threadIdx.x % XS, g = threadIdx.x / XS, x = blockIdx.x * XS + xl;
+  const double* p = part + x;
+  double acc[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  int tile = g;
+  for (; tile + 7 * G < ntiles; tile += 8 * G) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc[u] += p[(size_t)(tile + u * G) * nx];
+  }
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    if (tile + u * G < ntiles) acc[u] += p[(size_t)(tile + u * G) * nx];
+  tmp[threadIdx.x] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+  __syncthreads();
+  if (threadIdx.x < XS) {
+    double s = 0.0;
+    for (int i = 0; i < G; ++i) s += tmp[i * XS + xl];
+    out[x] = s;
+  }
+}
+
+// the end of a run of steps: e <- E of the last one, and its series (or null)
+__global__ __launch_bounds__(kFT) void k_finish(const double* e_last, const double* driver, int nx, double* e,
+                                                 double* series) {
+  __shared__ double rs[8];
+  VPFP_CTX;
+  for (int x = c.tid; x < nx; x += kFT) e[x] = e_last[x];
+  if (series) vp::series_body<kFT>(c, e_last, driver, nx, series, rs);
 }
 
 template <class T>
@@ -198,15 +231,8 @@ int launch_field(const vp::FieldArgs& a, hipStream_t s, int n_inst) {
   using Cfg = vp::FieldCfg<M, Q, kFT>;
   auto kern = k_field<M, Q>;
   if (int rc = set_lds(kern, Cfg::lds)) return rc;
-  vp::FieldArgs b = a;
-  int xm_blocks = 0;
-  if (b.xm_out) {
-    if (n_inst > 0) return fail(VPFP_EBADARG, "x-modes ride only on a single-grid field launch");
-    b.xm_blk0 = field_grid(a.nx);
-    xm_blocks = (b.xm_n * b.xm_nv + kFT - 1) / kFT;
-  }
-  const dim3 grid = n_inst > 0 ? dim3(1, n_inst) : dim3(field_grid(a.nx) + xm_blocks);
-  hipLaunchKernelGGL(kern, grid, dim3(kFT), Cfg::lds, s, b);
+  const dim3 grid = n_inst > 0 ? dim3(1, n_inst) : dim3(field_grid(a.nx));
+  hipLaunchKernelGGL(kern, grid, dim3(kFT), Cfg::lds, s, a);
   return launched();
 }
 
@@ -370,7 +396,7 @@ struct vpfp_plan_s {
   bool nx_pow2 = false, nv_pow2 = false;
   int C = 0, ntiles = 0;
   int row_q = 0;   // values per thread of the row kernels (0: row-count rule)
-  int fuse = -1;   // field solved by the last drift workgroup: 1 yes, 0 no, -1 size rule
+  int fuse = -1;   // where the step solves the field (FieldMode), -1 by size
   int xcd = 1;     // drift tile order (xcd_block); never slower in the measured shapes
   int dtiles = 1;  // column tiles per drift workgroup
   int dft = 0;                // x-advection as real-DFT products on MFMA (FP32, nx 32 or 64)
@@ -384,7 +410,8 @@ struct vpfp_plan_s {
   void* tw_x = nullptr;          // cx<T> twiddle tables for nx
   cx<double>* tw_xs = nullptr;   // cx<double> twiddle tables for nx (field)
   cx<double>* tw_xd = nullptr;   // cx<double>[nx] full table (direct-DFT field)
-  void* fcopy = nullptr;         // [nx][nv] storage type: f after a step (vpfp_step_n_store's x-modes)
+  void* fcopy = nullptr;         // [2][nx][nv] storage type: f after a step (the store's x-modes)
+  double* green = nullptr;       // [nx] Green's function of the field solve (nx <= 4096)
   double* dens = nullptr;        // [max(ntiles,1)][nx]
   double* ering = nullptr;       // [2][nx]
   double* rho_g = nullptr;       // [nx] field reduction scratch
@@ -561,13 +588,23 @@ int scan_tile(int nx, int nv) {
 }
 int scan_tiles_per_wg(long long tiles) { return tiles >= 4 * 2048 ? 4 : tiles >= 2 * 2048 ? 2 : 1; }
 
-// Field solve of the fused step: as a tail of the drift (its last workgroup)
-// or as a launch of its own.  The tail costs every drift workgroup a
-// device-scope release fence, which on this multi-XCD part writes back and
-// invalidates the L2 (buffer_wbl2 / buffer_inv); measured at nx = 64,
-// nv = 1024 the separate launch is faster (23.9 vs 26.0 us per step), so the
-// tail is left to the autotuner.
-bool default_fuse(int) { return false; }
+// Where the fused step solves the field (vpfp_tuning.fuse_field):
+//   kFieldLaunch  a launch of its own
+//   kFieldTail    the last drift workgroup.  It costs every drift workgroup a
+//                 device-scope release fence, which on this multi-XCD part
+//                 writes back and invalidates the L2 (buffer_wbl2 /
+//                 buffer_inv); the separate launch is faster
+//   kFieldRows    the row kernel, from the drift's partial density rows
+//   kFieldRowsSum the row kernel, from their sum by k_rho
+// Left at -1 the size decides between the last two (rule_mode): every row
+// workgroup reads all partial rows, so beyond kProSum values, or more columns
+// than its LDS holds, they are summed once first.
+enum FieldMode { kFieldLaunch = 0, kFieldTail = 1, kFieldRows = 2, kFieldRowsSum = 3 };
+constexpr int kFuseRowsNx = 128;  // fuse_field 2
+int rule_mode(vpfp_plan_t p) {
+  return p->nx <= vp::kProNx && (long long)p->ntiles * p->nx <= vp::kProSum ? kFieldRows : kFieldRowsSum;
+}
+int field_mode(vpfp_plan_t p) { return p->fuse >= 0 ? p->fuse : rule_mode(p); }
 
 enum KernelKind { KK_ROW = 0, KK_DRIFT = 1, KK_FIELD = 2, KK_OTHER = 3 };
 
@@ -676,6 +713,7 @@ vp::FieldArgs field_args(vpfp_plan_t p, const double* part, int ntiles, double s
   a.e_out2 = e_out2;
   a.series = series;
   a.series_stride = 0;
+  a.green = p->green;
   return a;
 }
 
@@ -712,11 +750,76 @@ int do_vdfdx(vpfp_plan_t p, const void* fin, void* fout, double dt, double* dens
   return drift_dispatch<T>(drift_args<T>(p, fin, fout, dt, dens), p->C, p->ntiles, s);
 }
 
+// one workgroup per row from 512 velocities on (100 x 1024 FP64: 8.4 us with one
+// wavefront per row, 2.8)
+template <class T>
+int launch_density(const void* f, int nx, int nv, double scale, double* part, hipStream_t s) {
+  const T* ft = reinterpret_cast<const T*>(f);
+  if (nv >= 512)
+    hipLaunchKernelGGL((k_density<T, 256>), dim3(nx), dim3(256), 0, s, ft, nx, nv, scale, part);
+  else
+    hipLaunchKernelGGL((k_density<T, 64>), dim3((nx + 3) / 4), dim3(256), 0, s, ft, nx, nv, scale, part);
+  return launched();
+}
+
 template <class T>
 int do_density(vpfp_plan_t p, const void* f, double scale, double* part, hipStream_t s) {
-  const int rows = 4;
-  hipLaunchKernelGGL(k_density<T>, dim3((p->nx + rows - 1) / rows), dim3(64 * rows), 0, s,
-                     reinterpret_cast<const T*>(f), p->nx, p->nv, scale, part);
+  return launch_density<T>(f, p->nx, p->nv, scale, part, s);
+}
+
+// the plan's field solves outside a step: any nx <= 4096
+int green_dispatch(const vp::FieldArgs& a, hipStream_t s) {
+  if (!a.green) return fail(VPFP_EUNSUPPORTED, "nx must be at most 4096 for the field solve");
+  hipLaunchKernelGGL(k_green, dim3((a.nx + 3) / 4), dim3(256), 0, s, a);
+  return launched();
+}
+
+// Where a step's field is formed: by the row kernel from the drift's partial
+// densities (field_rows), which k_rho sums first when they are too many for
+// every workgroup to read.  Returns the row kernel's field arguments.
+template <class T>
+int rows_field(vpfp_plan_t p, vp::RowArgs<T>* ra, const double* drv, double* e_out, bool sum, hipStream_t s) {
+  ra->field_pro = 1;
+  if (sum) {
+    const int XS = p->nx < kRhoXS ? p->nx : kRhoXS;
+    hipLaunchKernelGGL(k_rho, dim3(p->nx / XS), dim3(kFT), 0, s, p->dens, p->ntiles, p->nx, p->rho_g);
+    if (int rc = launched()) return rc;
+  }
+  ra->fld = field_args(p, sum ? p->rho_g : p->dens, sum ? 1 : p->ntiles, p->dv, drv, e_out, nullptr, nullptr, false);
+  return VPFP_OK;
+}
+
+// what a finished step leaves to the next row launch's extra workgroups
+template <class T>
+struct StepTail {
+  const double* e = nullptr;
+  const double* drv = nullptr;
+  double* series = nullptr;
+  const T* xm_f = nullptr;
+  cx<double>* xm_out = nullptr;
+  void attach(vpfp_plan_t p, vp::RowArgs<T>* ra, int n_modes) {
+    ra->prev_e = e;
+    ra->prev_drv = drv;
+    ra->prev_series = series;
+    ra->xm_f = xm_f;
+    ra->xm_n = n_modes;
+    ra->xm_tw = p->tw_xd;
+    ra->xm_out = xm_out;
+    *this = StepTail();
+  }
+};
+
+// the last step's tail and e <- E
+template <class T>
+int finish_steps(vpfp_plan_t p, const StepTail<T>& tail, int n_modes, const double* e_cur, double* e, hipStream_t s) {
+  if (tail.xm_out) {
+    if (int rc = prof_mark(p->prof, KK_OTHER, s)) return rc;
+    hipLaunchKernelGGL(k_xmodes<T>, dim3((n_modes * p->nv + 255) / 256), dim3(256), 0, s, tail.xm_f, p->nx, p->nv,
+                       n_modes, p->tw_xd, tail.xm_out);
+    if (int rc = launched()) return rc;
+    if (int rc = prof_mark(p->prof, KK_OTHER, s)) return rc;
+  }
+  hipLaunchKernelGGL(k_finish, dim3(1), dim3(kFT), 0, s, e_cur, tail.drv, p->nx, e, tail.series);
   return launched();
 }
 
@@ -753,74 +856,67 @@ int do_tri(vpfp_plan_t p, const double* A, const double* B, const double* Cc, co
 // f_store (optional): per-step f store, written by the row kernel between
 // the collision and the next half kick; n_modes == 0: [n][nx][nv] copies of
 // f (type T), n_modes > 0: [n][n_modes][nv] complex128 x-modes of f, formed
-// from the row kernel's copy in p->fcopy by extra workgroups of the next
-// step's field launch (one k_xmodes launch after the last step, and per
-// step when the field is not a launch of its own)
+// from the row kernel's copies in p->fcopy (two, used in turn) by extra
+// workgroups of the next step's row launch (one k_xmodes launch after the last
+// step)
 template <class T>
 int do_step_n(vpfp_plan_t p, void* f, double* e, int n, const double* driver, double* e_hist, double* moments,
               double* series, hipStream_t s, void* f_store = nullptr, int n_modes = 0) {
+  if (n <= 0) return prof_collect(p->prof);
   const bool coll = p->nu > 0.0;
   const double half = 0.5 * p->dt;
+  const int mode = field_mode(p);
+  if (p->fuse == 2 && p->nx > kFuseRowsNx)
+    return fail(VPFP_EUNSUPPORTED, "field in the row kernel needs nx <= " + std::to_string(kFuseRowsNx));
   auto ra = row_args<T>(p, f, f);
   ra.e = e;
   ra.dt_a = half;
   ra.flags = vp::RK_KICK_A;
-  if (n > 0) PROF(KK_ROW, row_dispatch<T>(ra, s, p->row_q));
+  PROF(KK_ROW, row_dispatch<T>(ra, s, p->row_q));
   const double* e_cur = e;
-  // field: 0 own launch, 1 tail of the drift, 2 prologue of the row kernel
-  const int mode = p->fuse >= 0 ? p->fuse : (default_fuse(p->nx) ? 1 : 0);
-  if (mode == 2 && p->nx > vp::kProNx)
-    return fail(VPFP_EUNSUPPORTED, "field in the row kernel needs nx <= " + std::to_string(vp::kProNx));
+  StepTail<T> tail;
   for (int i = 0; i < n; ++i) {
     double* ei = e_hist ? e_hist + (size_t)i * p->nx : p->ering + (size_t)(i & 1) * p->nx;
     const double* drv = driver ? driver + (size_t)i * p->nx : nullptr;
     double* ser = series ? series + 2 * (size_t)i : nullptr;
-    auto fa = field_args(p, p->dens, p->ntiles, p->dv, drv, ei, nullptr, ser, true);
-    auto* modes = reinterpret_cast<cx<double>*>(f_store);
-    if (f_store && n_modes > 0 && mode == 0 && i > 0) {
-      fa.xm_f = p->fcopy;
-      fa.xm_f32 = sizeof(T) == 4;
-      fa.xm_n = n_modes;
-      fa.xm_nv = p->nv;
-      fa.xm_tw = p->tw_xd;
-      fa.xm_out = modes + (size_t)(i - 1) * n_modes * p->nv;
-    }
-    if (mode == 1) {
+    auto rb = row_args<T>(p, f, f);
+    tail.attach(p, &rb, n_modes);
+    if (mode == kFieldTail) {
       auto da = drift_args<T>(p, f, f, p->dt, p->dens);
       da.fuse_field = 1;
-      da.fld = fa;
+      da.fld = field_args(p, p->dens, p->ntiles, p->dv, drv, ei, nullptr, ser, true);
       PROF(KK_DRIFT, drift_dispatch<T>(da, p->C, p->ntiles, s));
     } else {
       PROF(KK_DRIFT, (do_vdfdx<T>(p, f, f, p->dt, p->dens, s)));
-      if (mode == 0) PROF(KK_FIELD, field_dispatch(fa, true, s));
+      if (mode == kFieldLaunch) {
+        const auto fa = field_args(p, p->dens, p->ntiles, p->dv, drv, ei, nullptr, ser, true);
+        PROF(KK_FIELD, field_dispatch(fa, true, s));
+      } else if (mode == kFieldRowsSum) {
+        PROF(KK_FIELD, rows_field(p, &rb, drv, ei, true, s));
+      } else {
+        if (int rc = rows_field(p, &rb, drv, ei, false, s)) return rc;
+      }
     }
     e_cur = ei;
-    auto rb = row_args<T>(p, f, f);
     rb.e = e_cur;
-    if (mode == 2) {
-      rb.field_pro = 1;
-      rb.fld = field_args(p, p->dens, p->ntiles, p->dv, drv, ei, nullptr, ser, false);
-    }
     rb.dt_a = half;
     rb.dt_b = half;
     rb.moments = moments ? moments + (size_t)i * vp::kMoments * p->nx : nullptr;
     rb.flags = vp::RK_KICK_A | (coll ? vp::RK_COLLIDE : 0) | (moments ? vp::RK_MOMENTS : 0) |
                (i + 1 < n ? vp::RK_KICK_B : 0);
     if (f_store)
-      rb.f_copy = n_modes > 0 ? reinterpret_cast<T*>(p->fcopy)
+      rb.f_copy = n_modes > 0 ? reinterpret_cast<T*>(p->fcopy) + (size_t)(i & 1) * p->nx * p->nv
                               : reinterpret_cast<T*>(f_store) + (size_t)i * p->nx * p->nv;
     PROF(KK_ROW, row_dispatch<T>(rb, s, p->row_q));
-    if (f_store && n_modes > 0 && (mode != 0 || i + 1 == n)) {
-      const int total = n_modes * p->nv;
-      if (int rc = prof_mark(p->prof, KK_OTHER, s)) return rc;
-      hipLaunchKernelGGL(k_xmodes<T>, dim3((total + 255) / 256), dim3(256), 0, s,
-                         reinterpret_cast<const T*>(p->fcopy), p->nx, p->nv, n_modes, p->tw_xd,
-                         modes + (size_t)i * n_modes * p->nv);
-      if (int rc = launched()) return rc;
-      if (int rc = prof_mark(p->prof, KK_OTHER, s)) return rc;
+    tail.e = ei;
+    tail.drv = drv;
+    tail.series = mode >= kFieldRows ? ser : nullptr;
+    if (f_store && n_modes > 0) {
+      tail.xm_f = rb.f_copy;
+      tail.xm_out = reinterpret_cast<cx<double>*>(f_store) + (size_t)i * n_modes * p->nv;
     }
   }
-  if (n > 0) VPFP_HIP(hipMemcpyAsync(e, e_cur, sizeof(double) * p->nx, hipMemcpyDeviceToDevice, s));
+  if (int rc = finish_steps(p, tail, n_modes, e_cur, e, s)) return rc;
   return prof_collect(p->prof);
 }
 
@@ -864,13 +960,17 @@ template <class T>
 int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const double* driver, double* e_hist,
                    double* moments, double* series, hipStream_t s, void* f_store, int n_modes) {
   const std::vector<Stage> st = scheme_stages(scheme, p->dt);
+  if (n <= 0) return prof_collect(p->prof);
   const int ns = (int)st.size();
   const bool coll = p->nu > 0.0;
   const bool first_kick = st[0].kick, last_kick = st[ns - 1].kick;
-  auto* modes = reinterpret_cast<cx<double>*>(f_store);
+  // every field solve is formed by the row launch that follows it, by the size
+  // rule (the tuning's other forms are for the leapfrog step)
+  const bool sum = rule_mode(p) == kFieldRowsSum;
   const double* e_cur = e;
   long long field_no = 0;
-  if (n > 0 && first_kick) {
+  StepTail<T> tail;
+  if (first_kick) {
     auto ra = row_args<T>(p, f, f);
     ra.e = e;
     ra.dt_a = st[0].c * p->dt;
@@ -879,29 +979,33 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
   }
   for (int i = 0; i < n; ++i) {
     int j = 0;  // field solve of this step
+    vp::RowArgs<T> next = row_args<T>(p, f, f);  // the next row launch, with the field it forms
+    const double* drv = nullptr;
     for (int k = 0; k < ns; ++k) {
       const Stage& g = st[k];
       if (g.kick) {
         if (k == 0 || k == ns - 1) continue;  // fused into the row launch that ends a step
-        auto rk = row_args<T>(p, f, f);
-        rk.e = e_cur;
-        rk.dt_a = g.c * p->dt;
-        rk.flags = vp::RK_KICK_A;
-        PROF(KK_ROW, row_dispatch<T>(rk, s, p->row_q));
+        tail.attach(p, &next, n_modes);
+        next.e = e_cur;
+        next.dt_a = g.c * p->dt;
+        next.flags = vp::RK_KICK_A;
+        PROF(KK_ROW, row_dispatch<T>(next, s, p->row_q));
+        next = row_args<T>(p, f, f);
         continue;
       }
       PROF(KK_DRIFT, (do_vdfdx<T>(p, f, f, g.c * p->dt, p->dens, s)));
       const bool last = j == kSchemeFields - 1;
       double* eo = (last && e_hist) ? e_hist + (size_t)i * p->nx : p->ering + (size_t)(field_no & 1) * p->nx;
-      const double* drv = driver ? driver + ((size_t)i * kSchemeFields + j) * p->nx : nullptr;
-      double* ser = (last && series) ? series + 2 * (size_t)i : nullptr;
-      auto fa = field_args(p, p->dens, p->ntiles, p->dv, drv, eo, nullptr, ser, true);
-      PROF(KK_FIELD, field_dispatch(fa, true, s));
+      drv = driver ? driver + ((size_t)i * kSchemeFields + j) * p->nx : nullptr;
+      if (sum)
+        PROF(KK_FIELD, rows_field(p, &next, drv, eo, true, s));
+      else if (int rc = rows_field(p, &next, drv, eo, false, s))
+        return rc;
       e_cur = eo;
       ++j;
       ++field_no;
     }
-    auto rb = row_args<T>(p, f, f);
+    vp::RowArgs<T>& rb = next;
     rb.e = e_cur;
     rb.dt_a = last_kick ? st[ns - 1].c * p->dt : 0.0;
     rb.dt_b = st[0].c * p->dt;
@@ -909,20 +1013,23 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
     rb.flags = (last_kick ? vp::RK_KICK_A : 0) | (coll ? vp::RK_COLLIDE : 0) | (moments ? vp::RK_MOMENTS : 0) |
                (first_kick && i + 1 < n ? vp::RK_KICK_B : 0);
     if (f_store)
-      rb.f_copy = n_modes > 0 ? reinterpret_cast<T*>(p->fcopy)
+      rb.f_copy = n_modes > 0 ? reinterpret_cast<T*>(p->fcopy) + (size_t)(i & 1) * p->nx * p->nv
                               : reinterpret_cast<T*>(f_store) + (size_t)i * p->nx * p->nv;
-    if (rb.flags || rb.f_copy) PROF(KK_ROW, row_dispatch<T>(rb, s, p->row_q));
+    if (rb.flags || rb.f_copy) {
+      PROF(KK_ROW, row_dispatch<T>(rb, s, p->row_q));
+    } else {
+      // PEFRL without a collision or outputs ends with its field: no row launch
+      PROF(KK_FIELD, field_dispatch(field_args(p, p->dens, p->ntiles, p->dv, drv, rb.fld.e_out, nullptr, nullptr, true), true, s));
+    }
+    tail.e = e_cur;
+    tail.drv = drv;
+    tail.series = series ? series + 2 * (size_t)i : nullptr;
     if (f_store && n_modes > 0) {
-      const int total = n_modes * p->nv;
-      if (int rc = prof_mark(p->prof, KK_OTHER, s)) return rc;
-      hipLaunchKernelGGL(k_xmodes<T>, dim3((total + 255) / 256), dim3(256), 0, s,
-                         reinterpret_cast<const T*>(p->fcopy), p->nx, p->nv, n_modes, p->tw_xd,
-                         modes + (size_t)i * n_modes * p->nv);
-      if (int rc = launched()) return rc;
-      if (int rc = prof_mark(p->prof, KK_OTHER, s)) return rc;
+      tail.xm_f = rb.f_copy;
+      tail.xm_out = reinterpret_cast<cx<double>*>(f_store) + (size_t)i * n_modes * p->nv;
     }
   }
-  if (n > 0) VPFP_HIP(hipMemcpyAsync(e, e_cur, sizeof(double) * p->nx, hipMemcpyDeviceToDevice, s));
+  if (int rc = finish_steps(p, tail, n_modes, e_cur, e, s)) return rc;
   return prof_collect(p->prof);
 }
 
@@ -1208,9 +1315,10 @@ int autotune_plan(vpfp_plan_t p, int n_steps, hipStream_t s) {
   for (int q : row_q_candidates(p->nv, p->delta != 0))
     for (int C : {4, 8, 16, 32}) {
       if (C > p->nv) continue;
-      for (int fuse : {0, 1, 2}) {
+      for (int fuse : {0, 1, 2, -1}) {
         if (fuse == 1 && p->nx > 256) continue;
-        if (fuse == 2 && p->nx > vp::kProNx) continue;
+        if (fuse == -1 && p->nx <= kFuseRowsNx) continue;  // fuse 2 is the rule's choice there
+        if (fuse == 2 && p->nx > kFuseRowsNx) continue;
         for (int xo : {0, 1})
           for (int dt : {1, 2, 4}) {
             // more tiles per workgroup only where it changes the grid
@@ -1740,6 +1848,17 @@ int vpfp_plan_create(const vpfp_grid_desc* d, vpfp_plan_t* out) {
   if (!rc) rc = dalloc(p, &p->series, 2 * sizeof(double));
   if (!rc) rc = dalloc(p, &p->rho_g, nxb);
   if (!rc) rc = dalloc(p, &p->counter, 64);
+  if (!rc && p->nx <= 4096) {
+    rc = dalloc(p, &p->green, nxb);
+    if (!rc) {
+      hipLaunchKernelGGL(k_green_table, dim3((p->nx + 3) / 4), dim3(256), 0, 0, p->okx, p->tw_xd, p->nx, p->green);
+      rc = launched();
+    }
+    if (!rc) {
+      hipError_t e = hipStreamSynchronize(0);
+      if (e != hipSuccess) rc = fail(VPFP_EHIP, std::string("hipStreamSynchronize: ") + hipGetErrorString(e));
+    }
+  }
   if (!rc) {
     hipError_t e = hipMemset(p->counter, 0, 64);
     if (e != hipSuccess) rc = fail(VPFP_EHIP, std::string("hipMemset: ") + hipGetErrorString(e));
@@ -1814,9 +1933,7 @@ int vpfp_solve_for_field(vpfp_plan_t p, const double* n, double* e_out, void* st
   if (int rc = check_plan(p)) return rc;
   if (!n || !e_out) return fail(VPFP_EBADARG, "null array");
   if (p->nx < 2) return fail(VPFP_EUNSUPPORTED, "nx must be at least 2");
-  const bool pow2 = p->nx_pow2 && p->nx >= 4 && p->nx <= 4096;
-  auto fa = field_args(p, n, 1, 1.0, nullptr, e_out, nullptr, nullptr, pow2);
-  return field_dispatch(fa, pow2, p->streams.use(stream));
+  return green_dispatch(field_args(p, n, 1, 1.0, nullptr, e_out, nullptr, nullptr, false), p->streams.use(stream));
 }
 
 int vpfp_field(vpfp_plan_t p, const void* f, const double* driver, double* e_out, void* stream) {
@@ -1825,9 +1942,7 @@ int vpfp_field(vpfp_plan_t p, const void* f, const double* driver, double* e_out
   int rc = p->prec == VPFP_F64 ? do_density<double>(p, f, p->dv, p->dens, p->streams.use(stream))
                                : do_density<float>(p, f, p->dv, p->dens, p->streams.use(stream));
   if (rc) return rc;
-  const bool pow2 = p->nx_pow2 && p->nx >= 4 && p->nx <= 4096;
-  auto fa = field_args(p, p->dens, 1, 1.0, driver, e_out, nullptr, nullptr, pow2);
-  return field_dispatch(fa, pow2, p->streams.use(stream));
+  return green_dispatch(field_args(p, p->dens, 1, 1.0, driver, e_out, nullptr, nullptr, false), p->streams.use(stream));
 }
 
 int vpfp_field_noalloc(int nx, int nv, int precision, double dv, const double* one_over_kx, const void* f,
@@ -1851,14 +1966,9 @@ int vpfp_field_noalloc(int nx, int nv, int precision, double dv, const double* o
   hipLaunchKernelGGL(k_twiddles, dim3((entries + 255) / 256), dim3(256), 0, s, tw, nx, split);
   if (int rc = launched()) return rc;
   // n(x) = dv * trapz row sums: every entry is written before it is read
-  const int rows = 4;
-  if (precision == VPFP_F64)
-    hipLaunchKernelGGL(k_density<double>, dim3((nx + rows - 1) / rows), dim3(64 * rows), 0, s,
-                       reinterpret_cast<const double*>(f), nx, nv, dv, dens);
-  else
-    hipLaunchKernelGGL(k_density<float>, dim3((nx + rows - 1) / rows), dim3(64 * rows), 0, s,
-                       reinterpret_cast<const float*>(f), nx, nv, dv, dens);
-  if (int rc = launched()) return rc;
+  if (int rc = precision == VPFP_F64 ? launch_density<double>(f, nx, nv, dv, dens, s)
+                                     : launch_density<float>(f, nx, nv, dv, dens, s))
+    return rc;
   vp::FieldArgs a;
   std::memset(&a, 0, sizeof(a));
   a.part = dens;
@@ -2357,7 +2467,7 @@ int vpfp_step_n_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, con
   if (int rc = need_spectral_x(p)) return rc;
   if (p->nx > 2048) return fail(VPFP_EUNSUPPORTED, "nx too large for the fused step");
   if (n_modes > 0 && !p->fcopy) {
-    if (int rc = dalloc(p, &p->fcopy, (size_t)p->nx * p->nv * (p->prec == VPFP_F64 ? 8 : 4))) return rc;
+    if (int rc = dalloc(p, &p->fcopy, 2 * (size_t)p->nx * p->nv * (p->prec == VPFP_F64 ? 8 : 4))) return rc;
   }
   return p->prec == VPFP_F64
              ? do_step_scheme<double>(p, scheme, f, e, n, driver, e_hist, moments, series, p->streams.use(stream),
@@ -2376,7 +2486,7 @@ int vpfp_step_n_store(vpfp_plan_t p, void* f, double* e, int n, const double* dr
   if (int rc = need_spectral_x(p)) return rc;
   if (p->nx > 2048) return fail(VPFP_EUNSUPPORTED, "nx too large for the fused step");
   if (n_modes > 0 && !p->fcopy) {
-    if (int rc = dalloc(p, &p->fcopy, (size_t)p->nx * p->nv * (p->prec == VPFP_F64 ? 8 : 4))) return rc;
+    if (int rc = dalloc(p, &p->fcopy, 2 * (size_t)p->nx * p->nv * (p->prec == VPFP_F64 ? 8 : 4))) return rc;
   }
   return p->prec == VPFP_F64
              ? do_step_n<double>(p, f, e, n, driver, e_hist, moments, series, p->streams.use(stream), f_store, n_modes)

@@ -166,13 +166,7 @@ struct FieldArgs {
   double* e_out2;         // [nx] or null
   double* series;         // [2] or null: mean(E^2), mean(driver^2)
   int series_stride;      // batched scan: doubles between consecutive instances' series entries
-  // single grid (vpfp_step_n_store): workgroups xm_blk0 and up of the launch
-  // form the first xm_n x-modes of xm_f [nx][xm_nv] (FP32 if xm_f32, else
-  // FP64) into xm_out [xm_n][xm_nv] (xmodes_body); xm_tw[r] = exp(-2 pi i r / nx)
-  const void* xm_f;
-  int xm_f32, xm_n, xm_nv, xm_blk0;
-  const cx<double>* xm_tw;
-  cx<double>* xm_out;
+  const double* green;    // [nx] Green's function of the solve (single grids; field_rows, green_body)
 };
 
 // The view of instance inst of a batched field solve: every array is
@@ -196,7 +190,7 @@ VP_HD FieldArgs field_instance(const FieldArgs& a, int inst) {
 
 // rho[x] = 1 - scale * sum_tiles part[tile][x] for x in [x0, x0 + XS)
 // (all FT threads; XS divides FT or FT divides XS)
-template <int FT, bool COH = false, class Ctx>
+template <int FT, bool COH = false, int U = 8, class Ctx>
 VP_HD void field_density(Ctx& c, const FieldArgs& a, int x0, int XS, double* rho, double* tmp) {
   const int nx = a.nx;
   const int G = XS >= FT ? 1 : FT / XS;
@@ -204,15 +198,23 @@ VP_HD void field_density(Ctx& c, const FieldArgs& a, int x0, int XS, double* rho
     const int xl = l0 % XS, g = l0 / XS;
     const double* p = a.part + x0 + xl;
     auto ld = [&](int tl) { return COH ? c.load_coherent(p + (size_t)tl * nx) : p[(size_t)tl * nx]; };
-    // eight independent partial sums keep eight loads in flight per thread
-    double acc[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    int tile = g;
-    for (; tile + 7 * G < a.ntiles; tile += 8 * G) {
+    // U independent partial sums keep U loads in flight per thread
+    double acc[U];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) acc[u] += ld(tile + u * G);
+    for (int u = 0; u < U; ++u) acc[u] = 0.0;
+    int tile = g;
+    for (; tile + (U - 1) * G < a.ntiles; tile += U * G) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc[u] += ld(tile + u * G);
     }
-    for (int u = 0; tile < a.ntiles; tile += G, ++u) acc[u & 7] += ld(tile);
-    tmp[l0] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (tile + u * G < a.ntiles) acc[u] += ld(tile + u * G);
+#pragma unroll
+    for (int h = U / 2; h >= 1; h >>= 1)
+#pragma unroll
+      for (int u = 0; u < h; ++u) acc[u] += acc[u + h];
+    tmp[l0] = acc[0];
   }
   c.sync();
   for (int xl = c.tid; xl < XS; xl += FT) {
@@ -223,98 +225,121 @@ VP_HD void field_density(Ctx& c, const FieldArgs& a, int x0, int XS, double* rho
   c.sync();
 }
 
-// Field at a workgroup's own rows from the drift's partial density rows, by
-// the direct DFT of field_dft_body (small single grids, nx <= kProNx):
-//   E(x) = Re sum_m F_m exp(2 pi i m x / nx) / nx + driver(x),
-//   F_m = i g_m sum_j rho_j exp(-2 pi i m j / nx), g_m = (okx_m - okx_{nx-m}) / 2.
-// Every workgroup forms all nx values of E (each sum split over P = FT/nx
-// adjacent lanes, joined by shuffles), writes those of rows [row0, row0 +
-// nrows) to e_out (and e_out2); the workgroup holding row 0 writes the
-// series.  All FT threads call it; erow (= lds + ProCfg::erow_off) holds E.
-// lds: tw [kProNx] cx | okx [kProNx] | rho [kProNx] | F [kProNx] cx | tmp [tmp_n] | E [kProNx]
-constexpr int kProNx = 128;
+// Field at a workgroup's own rows (single grids): with the Green's function
+//   g_d = (1/nx) sum_m Re(i okx_m exp(2 pi i m d / nx))
+// of the solve, formed once per plan, E(x) = driver(x) + sum_j g_{x-j} rho_j is
+// one dot product per row, so a row needs no field launch and no transform
+// between the drift and its kick.  The partial density rows are summed here
+// when they are few (kProSum values, nx <= kProNx: every workgroup reads them
+// all), otherwise by k_rho into one row (ntiles = 1).  Every thread of a row
+// gets E; thread t = 0 writes it.  64 x 1024 FP64 step: 21.2 us with the field
+// launch, 18.2 with this; 1024 x 8192 (summed by k_rho): 187 -> 175.
+// lds: rho [kProNx] | tmp [max(kProNx, FT)] | row_sum scratch [16]
+constexpr int kProNx = 256;
+constexpr int kProSum = 8192;
 template <int FT>
 struct ProCfg {
-  static constexpr int tmp_n = 2 * kProNx > FT ? 2 * kProNx : FT;
-  static constexpr int tw_off = 0;
-  static constexpr int okx_off = tw_off + kProNx * 16;
-  static constexpr int rho_off = okx_off + kProNx * 8;
-  static constexpr int f_off = rho_off + kProNx * 8;
-  static constexpr int tmp_off = f_off + kProNx * 16;
-  static constexpr int erow_off = tmp_off + tmp_n * 8;
-  static constexpr int bytes = erow_off + kProNx * 8;
+  static constexpr int tmp_n = kProNx > FT ? kProNx : FT;
+  static constexpr int bytes = (kProNx + tmp_n + 16) * 8;
 };
 
-template <int FT, class Ctx>
-VP_HD void field_rows(Ctx& c, const FieldArgs& a, unsigned char* lds, int row0, int nrows) {
-  using P_ = ProCfg<FT>;
+template <int FT, int TPT, class Ctx>
+VP_HD double field_rows(Ctx& c, const FieldArgs& a, unsigned char* lds, int row, bool valid, int t) {
+  double* rho = reinterpret_cast<double*>(lds);
+  double* tmp = rho + kProNx;
+  double* rs = tmp + ProCfg<FT>::tmp_n;
   const int nx = a.nx;
-  cx<double>* twl = reinterpret_cast<cx<double>*>(lds + P_::tw_off);
-  double* okx = reinterpret_cast<double*>(lds + P_::okx_off);
-  double* rho = reinterpret_cast<double*>(lds + P_::rho_off);
-  cx<double>* F = reinterpret_cast<cx<double>*>(lds + P_::f_off);
-  double* tmp = reinterpret_cast<double*>(lds + P_::tmp_off);
-  double* E = reinterpret_cast<double*>(lds + P_::erow_off);
-  for (int i = c.tid; i < nx; i += FT) {
-    twl[i] = a.tw[i];
-    okx[i] = a.okx[i];
+  double s[1] = {0.0};
+  if (a.ntiles == 1) {
+#pragma unroll 4
+    for (int j = t; j < nx; j += TPT) s[0] += a.green[(row - j) & (nx - 1)] * (1.0 - a.scale * a.part[j]);
+  } else {
+    field_density<FT, false, 16>(c, a, 0, nx, rho, tmp);  // ends with a barrier
+    for (int j = t; j < nx; j += TPT) s[0] += a.green[(row - j) & (nx - 1)] * rho[j];
   }
-  field_density<FT>(c, a, 0, nx, rho, tmp);  // ends with a barrier
-  // P lanes per output: the largest power of two <= FT / nx, at most 64
-  int P = 1;
-  while (2 * P * nx <= FT && P < 64) P *= 2;
-  const int part = c.tid % P;
-  const int G = FT / P;                  // outputs per round
-  const int rounds = (nx + G - 1) / G;   // the same for every thread
-  for (int rd = 0; rd < rounds; ++rd) {
-    const int m0 = c.tid / P + rd * G;
-    const int m = m0 < nx ? m0 : nx - 1;
-    cx<double> s = mk<double>(0.0, 0.0);
-    for (int j = part; j < nx; j += P) {
-      const cx<double> w = twl[(int)(((long long)m * j) % nx)];
-      s.re += rho[j] * w.re;
-      s.im += rho[j] * w.im;
-    }
-    for (int o = 1; o < P; o <<= 1) {
-      s.re += c.shfl_xor(s.re, o, P);
-      s.im += c.shfl_xor(s.im, o, P);
-    }
-    if (part == 0 && m0 < nx) {
-      const double g = 0.5 * (okx[m] - okx[(nx - m) % nx]);
-      F[m] = mk<double>(-g * s.im, g * s.re);
-    }
+  row_sum<TPT, 1>(c, s, rs);
+  if constexpr (TPT <= 64) c.sync();  // rho read before the transforms take the LDS
+  const double e = s[0] + (a.driver ? a.driver[row] : 0.0);
+  if (valid && t == 0) {
+    a.e_out[row] = e;
+    if (a.e_out2) a.e_out2[row] = e;
   }
-  c.sync();
-  for (int rd = 0; rd < rounds; ++rd) {
-    const int x0 = c.tid / P + rd * G;
-    const int x = x0 < nx ? x0 : nx - 1;
-    double s = 0.0;
-    for (int m = part; m < nx; m += P) {
-      const cx<double> w = twl[(int)(((long long)m * x) % nx)];
-      s += F[m].re * w.re + F[m].im * w.im;
-    }
-    for (int o = 1; o < P; o <<= 1) s += c.shfl_xor(s, o, P);
-    if (part == 0 && x0 < nx) E[x] = s / nx + (a.driver ? a.driver[x] : 0.0);
+  return e;
+}
+
+// mean(E^2) and mean(driver^2) of a finished step (one workgroup of FT threads)
+template <int FT, class Ctx>
+VP_HD void series_body(Ctx& c, const double* e, const double* driver, int nx, double* out, double* rs) {
+  double acc[2] = {0.0, 0.0};
+  for (int x = c.tid; x < nx; x += FT) {
+    const double ex = e[x], dr = driver ? driver[x] : 0.0;
+    acc[0] += ex * ex;
+    acc[1] += dr * dr;
   }
-  c.sync();
-  for (int r = c.tid; r < nrows; r += FT) {
-    a.e_out[row0 + r] = E[row0 + r];
-    if (a.e_out2) a.e_out2[row0 + r] = E[row0 + r];
+  row_sum<FT, 2>(c, acc, rs);
+  if (c.tid == 0) {
+    out[0] = acc[0] / nx;
+    out[1] = acc[1] / nx;
   }
-  if (row0 == 0 && a.series) {
-    double acc[2] = {0.0, 0.0};
-    for (int x = c.tid; x < nx; x += FT) {
-      const double dr = a.driver ? a.driver[x] : 0.0;
-      acc[0] += E[x] * E[x];
-      acc[1] += dr * dr;
-    }
-    row_sum<FT, 2>(c, acc, tmp);
-    if (c.tid == 0) {
-      a.series[0] = acc[0] / nx;
-      a.series[1] = acc[1] / nx;
-    }
+}
+
+// E(x) = driver(x) + sum_j g_{x-j} rho_j at any nx, one wavefront per x (the
+// plan's own field solves): nx = 100 2.7 us where the direct transform on one
+// workgroup took 22.5
+template <class Ctx>
+VP_HD void green_body(Ctx& c, const FieldArgs& a) {
+  const int lane = c.tid & 63;
+  const int x0 = c.bid * (c.nthr / 64) + (c.tid >> 6);
+  const int x = x0 < a.nx ? x0 : a.nx - 1;
+  double s = 0.0;
+#pragma unroll 4
+  for (int j = lane; j < a.nx; j += 64) {
+    const int d = x - j;
+    s += a.green[d < 0 ? d + a.nx : d] * (1.0 - a.scale * a.part[j]);
   }
-  c.sync();
+  s = lane_sum<64>(c, s);
+  if (x0 < a.nx && lane == 0) a.e_out[x] = s + (a.driver ? a.driver[x] : 0.0);
+}
+
+// g_d, one wavefront per d: the bins m and nx - m of the sum are equal (only the
+// odd part (okx_m - okx_{nx-m}) / 2 of the multiplier reaches the real part), so
+// g_d = -(2/nx) sum_{0 < m < nx/2} g_m sin(2 pi m d / nx); tw[n] = exp(-2 pi i n / nx)
+template <class Ctx>
+VP_HD void green_table_body(Ctx& c, const double* okx, const cx<double>* tw, int nx, double* green) {
+  const int lane = c.tid & 63;
+  const int d0 = c.bid * (c.nthr / 64) + (c.tid >> 6);
+  const int d = d0 < nx ? d0 : nx - 1;
+  double s = 0.0;
+  for (int m = 1 + lane; 2 * m < nx; m += 64)
+    s += 0.5 * (okx[m] - okx[nx - m]) * tw[(int)(((long long)m * d) % nx)].im;
+  s = lane_sum<64>(c, s);
+  if (d0 < nx && lane == 0) green[d] = 2.0 * s / nx;
+}
+
+// ---------------------------------------------------------------------------
+// first nm Fourier modes along x of every v column:
+//   out[m][v] = sum_x f(x, v) exp(-2 pi i m x / nx)     (step.py:130-135)
+// one thread per (m, v); the x sum is sequential in x order
+// ---------------------------------------------------------------------------
+template <class T, class Ctx>
+VP_HD void xmodes_body(Ctx& c, const T* f, int nx, int nv, int nm, const cx<double>* tw, cx<double>* out) {
+  const int idx = c.bid * c.nthr + c.tid;
+  if (idx >= nm * nv) return;
+  const int m = idx / nv, col = idx % nv;
+  double re = 0.0, im = 0.0;
+  // r = m x mod nx by increments: the loads of f and of the twiddles do not
+  // wait on an index division, so consecutive iterations overlap
+  int r = 0;
+#pragma unroll 16
+  for (int x = 0; x < nx; ++x) {
+    const cx<double> w = tw[r];
+    const double fv = (double)f[(size_t)x * nv + col];
+    re += fv * w.re;
+    im += fv * w.im;
+    r += m;
+    if (r >= nx) r -= nx;
+  }
+  out[idx] = mk<double>(re, im);
 }
 
 // ---------------------------------------------------------------------------
@@ -339,9 +364,19 @@ struct RowArgs {
   const double* nu_dt_inst;  // batched scan: nu*dt per instance (rows are instance-major), or null
   int rows_per_inst;         // x rows per instance in a batch
   // field in the prologue (field_rows): E of the workgroup's rows from the
-  // drift's partial densities instead of e (single grid, nx <= kProNx)
+  // drift's densities instead of e (single grid)
   int field_pro;
   FieldArgs fld;
+  // extra workgroups after the rows' own, for a finished earlier step (single
+  // grid): one for the series of its E and driver (prev_series), then
+  // xm_n * xm_nv threads for the first xm_n x-modes of its f copy xm_f [nx][nv]
+  const double* prev_e;
+  const double* prev_drv;
+  double* prev_series;
+  const T* xm_f;
+  int xm_n;
+  const cx<double>* xm_tw;  // exp(-2 pi i r / nx)
+  cx<double>* xm_out;       // [xm_n][nv]
   // delta-f storage: f holds f - B(v) for a fixed background B (bg [nv],
   // FP64; spectrum tables bg_hat [nv] of BgPhaseMul in the storage precision);
   // the kicks shift B spectrally as part of the deviation's multiply, the
@@ -378,6 +413,19 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
   using Cfg = RowCfg<T, M, Q>;
   constexpr int TPT = Cfg::TPT;
   constexpr int L = Cfg::L;
+  if (a.prev_series || a.xm_out) {
+    int b = c.bid - (a.nx + Cfg::rows - 1) / Cfg::rows;
+    if (b >= 0 && a.prev_series && b-- == 0) {
+      series_body<Cfg::wg>(c, a.prev_e, a.prev_drv, a.nx, a.prev_series, reinterpret_cast<double*>(lds));
+      return;
+    }
+    if (b >= 0) {
+      Ctx x = c;
+      x.bid = b;
+      xmodes_body<T>(x, a.xm_f, a.nx, a.nv, a.xm_n, a.xm_tw, a.xm_out);
+      return;
+    }
+  }
   const int t = c.tid % TPT;
   const int rl = c.tid / TPT;
   const int row = c.bid * Cfg::rows + rl;
@@ -393,11 +441,7 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
   for (int i = 0; i < Q; ++i) v[i] = src[t + i * TPT];
   double e = 0.0;
   if (a.field_pro) {
-    const int row0 = c.bid * Cfg::rows;
-    const int nr = a.nx - row0 < Cfg::rows ? a.nx - row0 : Cfg::rows;
-    field_rows<Cfg::wg>(c, a.fld, lds, row0, nr);
-    e = reinterpret_cast<const double*>(lds + ProCfg<Cfg::wg>::erow_off)[valid ? row : 0];
-    c.sync();  // every thread has its E before the transforms overwrite the prologue's LDS
+    e = field_rows<Cfg::wg, TPT>(c, a.fld, lds, rowc, valid, t);
   } else if (a.flags & (RK_KICK_A | RK_KICK_B)) {
     e = a.e[rowc];
   }
@@ -989,44 +1033,30 @@ VP_HD void drift_dft_body(Ctx& c, unsigned char* lds, const DriftArgs<float>& a)
 }
 
 // ---------------------------------------------------------------------------
-// density rows: part[x] = scale * sum_v w_v f(x, v)   (one wavefront per row)
+// density rows: part[x] = scale * sum_v w_v f(x, v), W threads per row (64: one
+// wavefront each, 256: one workgroup, for long rows), eight loads in flight
+// per thread
 // ---------------------------------------------------------------------------
-template <class T, class Ctx>
-VP_HD void density_body(Ctx& c, const T* f, int nx, int nv, double scale, double* part) {
-  const int lane = c.tid & 63;
-  const int row = c.bid * (c.nthr / 64) + (c.tid >> 6);
+template <class T, int W, class Ctx>
+VP_HD void density_body(Ctx& c, const T* f, int nx, int nv, double scale, double* part, double* rs) {
+  const int t = c.tid % W;
+  const int row = c.bid * (c.nthr / W) + c.tid / W;
   const int rowc = row < nx ? row : nx - 1;
   const T* fr = f + (size_t)rowc * nv;
   double s[1] = {0.0};
-  for (int m = lane; m < nv; m += 64) s[0] += trapw(m, nv) * (double)fr[m];
-  s[0] = lane_sum<64>(c, s[0]);
-  if (row < nx && lane == 0) part[row] = scale * s[0];
-}
-
-// ---------------------------------------------------------------------------
-// first nm Fourier modes along x of every v column:
-//   out[m][v] = sum_x f(x, v) exp(-2 pi i m x / nx)     (step.py:130-135)
-// one thread per (m, v); the x sum is sequential in x order
-// ---------------------------------------------------------------------------
-template <class T, class Ctx>
-VP_HD void xmodes_body(Ctx& c, const T* f, int nx, int nv, int nm, const cx<double>* tw, cx<double>* out) {
-  const int idx = c.bid * c.nthr + c.tid;
-  if (idx >= nm * nv) return;
-  const int m = idx / nv, col = idx % nv;
-  double re = 0.0, im = 0.0;
-  // r = m x mod nx by increments: the loads of f and of the twiddles do not
-  // wait on an index division, so consecutive iterations overlap
-  int r = 0;
-#pragma unroll 16
-  for (int x = 0; x < nx; ++x) {
-    const cx<double> w = tw[r];
-    const double fv = (double)f[(size_t)x * nv + col];
-    re += fv * w.re;
-    im += fv * w.im;
-    r += m;
-    if (r >= nx) r -= nx;
+  int m = t;
+  for (; m + 7 * W < nv; m += 8 * W) {
+    double x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = (double)fr[m + u * W];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s[0] += trapw(m + u * W, nv) * x[u];
   }
-  out[idx] = mk<double>(re, im);
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    if (m + u * W < nv) s[0] += trapw(m + u * W, nv) * (double)fr[m + u * W];
+  row_sum<W, 1>(c, s, rs);
+  if (row < nx && t == 0) part[row] = scale * s[0];
 }
 
 // ---------------------------------------------------------------------------

@@ -26,7 +26,8 @@ int launch_row_q(const vp::RowArgs<T>& a, hipStream_t s) {
   using Cfg = vp::RowCfg<T, M, Q>;
   auto kern = k_row<T, M, Q, BG>;
   if (int rc = set_lds(kern, Cfg::lds)) return rc;
-  const int grid = (a.nx + Cfg::rows - 1) / Cfg::rows;
+  int grid = (a.nx + Cfg::rows - 1) / Cfg::rows + (a.prev_series ? 1 : 0);
+  if (a.xm_out) grid += (a.xm_n * a.nv + Cfg::wg - 1) / Cfg::wg;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(Cfg::wg), Cfg::lds, s, a);
   return launched();
 }

@@ -6,7 +6,7 @@ reference's temp_storage schema (outer_loop.py:149-215) with host numpy
 arrays, so the reference's storage manager and diagnostics can consume it.
 
 With exponential pushers and the spectral field solve, a batch of steps runs
-as one call of a fused device loop: vpfp_step_n_store for leapfrog (three
+as one call of a fused device loop: vpfp_step_n_store for leapfrog (two
 kernels per step, f resident in HBM, the per-step f store or its x-modes
 written by the row kernel), vpfp_step_n_scheme for PEFRL and the 6th-order
 splitting (their drifts, field solves and kicks as device launches, the
@@ -139,7 +139,7 @@ class _FusedInnerLoop:
     """Batches of (leapfrog, PEFRL or 6th-order) + collision + storage steps
     on the device.
 
-    One vpfp_step_n_store (leapfrog: three launches per step) or
+    One vpfp_step_n_store (leapfrog: two launches per step) or
     vpfp_step_n_scheme call per batch, then one synchronisation: the E
     history, the moments and the f store come back by asynchronous copies
     into page-locked host arrays that this stepper owns and puts into
