@@ -3,16 +3,15 @@
 //
 // Data layouts
 //   rows of f, x, y, target, dy: [rows][256] FP32
-//   stored activations a1..a3 and pre-activation gradients dz1..dz3:
-//     [rows][64][256] BF16, channel-major (v contiguous)
+//   stored activations a1..a3 and the pre-activation gradient dz2:
+//     [rows][256][64] BF16, position-major (channels contiguous), the order of
+//     the LDS tile
 //   LDS "position-major" tile of one row: [260][kP] BF16, row p+2 holds the
 //     64 channels at position p (rows 0, 1, 258, 259 are the zero padding),
 //     kP = 80 keeps every 8-channel group 16-byte aligned and the MFMA
 //     operand reads (16 positions x 16 bytes per lane group) free of LDS
 //     bank conflicts: with a 144-byte pitch (kP = 72) they measured 2-way
 //     conflicted on gfx950, with 160 bytes conflict-free
-//   LDS "channel-major" tile: [64][kQ] BF16, element p+2 of channel c at
-//     c*kQ + p + 2 (zero padding at 0, 1, 258, 259)
 //
 // MFMA v_mfma_f32_16x16x32_bf16 (D = A B + C, A 16x32, B 32x16): lane l
 // supplies A[l%16][8(l/16)+j] and B[8(l/16)+j][l%16] for j < 8 and holds
@@ -50,12 +49,11 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kNV = VPFC_NV, kCH = VPFC_CHANNELS, kKS = VPFC_KERNEL, kK = kCH * kKS;
 constexpr int kP = 80;          // position-major pitch (BF16)
-constexpr int kQ = 272;         // channel-major pitch (BF16): 16-byte rows, reads up to p + 2 + 15 < 272
-constexpr int kQs = 266;        // channel-major pitch for 2-byte column reads (133 dwords: odd)
 constexpr int kRowsP = kNV + 4;
 constexpr int oW1 = 0, oB1 = oW1 + kCH * kKS, oW2 = oB1 + kCH, oB2 = oW2 + kCH * kK, oW3 = oB2 + kCH,
               oB3 = oW3 + kCH * kK, oW4 = oB3 + kCH, oB4 = oW4 + kK, kParams = oB4 + 1;
 static_assert(kParams == VPFC_NPARAMS, "parameter layout");
+constexpr int kPart = (kParams + 3) & ~3;  // pitch of the partial gradients: 16-byte rows
 constexpr int kPartWG = 256;    // workgroups of the gradient kernels (rows strided over them)
 
 __device__ __forceinline__ float bfr(float x) { return (float)(bf16)x; }
@@ -105,18 +103,6 @@ __device__ __forceinline__ void zero_pad_p(bf16* P) {
   for (int i = threadIdx.x; i < 4 * kP; i += blockDim.x) {
     const int r = i / kP, row = r < 2 ? r : kNV + r;
     P[row * kP + i % kP] = (bf16)0.f;
-  }
-}
-
-// global channel-major BF16 row [64][256] -> position-major LDS tile
-__device__ __forceinline__ void stage_p(bf16* P, const bf16* src) {
-  const int p = threadIdx.x;  // 256 threads, one position each
-#pragma unroll
-  for (int c0 = 0; c0 < kCH; c0 += 8) {
-    bf16x8 v;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = src[(c0 + j) * kNV + p];
-    *reinterpret_cast<bf16x8*>(P + (p + 2) * kP + c0) = v;
   }
 }
 
@@ -193,32 +179,42 @@ __device__ __forceinline__ float tanh_act(float x) {
 }
 
 // tanh(acc + b) of accumulator tile nt (channels co0..co0+3 of lane (m, g),
-// position 16 nt + m) into P at pr = P + (m + 2) kP + co0 and, when training,
-// into the stored activations at gr = gout + (row kCH + co0) kNV + m
+// position 16 nt + m) into P at pr = P + (m + 2) kP + co0
 template <int NT>
-__device__ __forceinline__ void act_tile(const floatx4& acc, const float (&b)[4], bf16* pr, bf16* gr) {
+__device__ __forceinline__ void act_tile(const floatx4& acc, const float (&b)[4], bf16* pr) {
   bf16x4 o;
 #pragma unroll
   for (int j = 0; j < 4; ++j) o[j] = (bf16)tanh_act(acc[j] + b[j]);
   *reinterpret_cast<bf16x4*>(pr + 16 * NT * kP) = o;
-  if (gr) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) gr[j * kNV + 16 * NT] = o[j];
-  }
 }
 
 // act_tile over the 16 tiles of a 64 -> 64 layer
 template <int NT = 0>
-__device__ __forceinline__ void act_tiles(const floatx4* acc, const float (&b)[4], bf16* pr, bf16* gr) {
+__device__ __forceinline__ void act_tiles(const floatx4* acc, const float (&b)[4], bf16* pr) {
   if constexpr (NT < 16) {
-    act_tile<NT>(acc[NT], b, pr, gr);
-    act_tiles<NT + 1>(acc, b, pr, gr);
+    act_tile<NT>(acc[NT], b, pr);
+    act_tiles<NT + 1>(acc, b, pr);
+  }
+}
+
+// the 256 positions of the LDS tile to a stored row of activations, 16 bytes
+// per thread and pass (written by the lanes that form them instead, each
+// channel's 2 bytes on its own, the forward pass of 4096 training rows took
+// 194 us, with this 178)
+__device__ __forceinline__ void store_tile(const bf16* P, bf16* dst) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int i = threadIdx.x + 256 * u;
+    *reinterpret_cast<bf16x8*>(dst + 8 * i) = *reinterpret_cast<const bf16x8*>(P + ((i >> 3) + 2) * kP + 8 * (i & 7));
   }
 }
 
 // three waves per SIMD (<= 168 registers) to match the three workgroups the
 // LDS allows; left to itself the compiler takes 260 registers (one wave per
-// SIMD), which measured 2.4x slower at 262144 rows
+// SIMD), which measured 2.4x slower at 262144 rows.  TRAIN, the variant that
+// stores what the backward pass needs, is a kernel of its own: in one kernel
+// its addresses spilled 140 bytes and applying cost 4 % more
+template <bool TRAIN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_fwd(FwdArgs a) {
   extern __shared__ __align__(16) unsigned char lds[];
   bf16* P = reinterpret_cast<bf16*>(lds);
@@ -247,7 +243,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
       srow = sqrtf(block_sum(d * d, red) * (1.f / kNV) + 1e-30f);
     }
     const bf16 xb = (bf16)((a.in_scale / srow) * d);
-    if (a.xin) a.xin[ro + t] = xb;
+    if constexpr (TRAIN) a.xin[ro + t] = xb;
     // x[t] is entry k of the record of position t + 2 - k
 #pragma unroll
     for (int k = 0; k < kKS; ++k) {
@@ -261,15 +257,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
       // the zero padding row of P)
       const bf16x8 A1 = *reinterpret_cast<const bf16x8*>(g == 0 ? w1b + 8 * (16 * wave + m) : P);
       const float b[4] = {a.p[oB1 + co0], a.p[oB1 + co0 + 1], a.p[oB1 + co0 + 2], a.p[oB1 + co0 + 3]};
-      bf16* gr = a.a1 ? a.a1 + ((size_t)row * kCH + co0) * kNV + m : nullptr;
       const bf16* rec = P + (m + 2) * kP + kCH;
       floatx4 acc[16];
 #pragma unroll
       for (int nt = 0; nt < 16; ++nt)
         acc[nt] = mfma(A1, *reinterpret_cast<const bf16x8*>(rec + 16 * nt * kP), floatx4{0.f, 0.f, 0.f, 0.f});
-      act_tiles(acc, b, pr, gr);
+      act_tiles(acc, b, pr);
     }
     __syncthreads();
+    if constexpr (TRAIN) store_tile(P, a.a1 + (size_t)row * kCH * kNV);
     // layers 2 and 3: 64 -> 64, tanh, in place: every wave has its sums in
     // registers before any wave overwrites the tile.  The weight fragments are
     // reloaded per row (L2-resident): keeping both layers' in registers
@@ -277,25 +273,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     {
       bf16x8 A[10];
       load_a(a.w2, A);
-      mconv(P, A, [&](floatx4* acc, int c0, int mm) {
+      mconv(P, A, [&](floatx4* acc, int c0, int) {
         const float b[4] = {a.p[oB2 + c0], a.p[oB2 + c0 + 1], a.p[oB2 + c0 + 2], a.p[oB2 + c0 + 3]};
-        bf16* gr = a.a2 ? a.a2 + ((size_t)row * kCH + c0) * kNV + mm : nullptr;
         __syncthreads();
-        act_tiles(acc, b, pr, gr);
+        act_tiles(acc, b, pr);
       });
     }
     __syncthreads();
+    if constexpr (TRAIN) store_tile(P, a.a2 + (size_t)row * kCH * kNV);
     {
       bf16x8 A[10];
       load_a(a.w3, A);
-      mconv(P, A, [&](floatx4* acc, int c0, int mm) {
+      mconv(P, A, [&](floatx4* acc, int c0, int) {
         const float b[4] = {a.p[oB3 + c0], a.p[oB3 + c0 + 1], a.p[oB3 + c0 + 2], a.p[oB3 + c0 + 3]};
-        bf16* gr = a.a3 ? a.a3 + ((size_t)row * kCH + c0) * kNV + mm : nullptr;
         __syncthreads();
-        act_tiles(acc, b, pr, gr);
+        act_tiles(acc, b, pr);
       });
     }
     __syncthreads();
+    if constexpr (TRAIN) store_tile(P, a.a3 + (size_t)row * kCH * kNV);
     // layer 4: 64 -> 1, linear; every row of A is W4, so lane (m, g) sums
     // y at position 16 nt + m in all four accumulator slots
     {
@@ -333,7 +329,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     }
     if (a.y_out) a.y_out[ro + t] = y;
     if (a.f_out) a.f_out[ro + t] = fv + (a.out_scale * srow) * y;
-    if (a.dy) {
+    if constexpr (TRAIN) {
       const float e = y - a.target[ro + t] / srow;
       a.dy[ro + t] = a.gscale * e;
       const float s = block_sum(e * e, red);
@@ -343,262 +339,392 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   }
 }
 // ----------------------------------------------------------------------------
-// backward through a 64 -> 64 layer (input gradient):
-//   dzp[ci][p] = bf16( (sum_{k', co} Wt[ci][k'*64 + co] dz[co][p + k' - 2]) (1 - ap[ci][p]^2) )
-// with Wt[ci][k'*64 + co] = W[co][(4 - k')*64 + ci] (flipped, transposed)
+// backward: two kernels, rows strided over the workgroups (512 threads)
+//
+// k_bwd_out: output layer and layer 3.  dz3 is formed from dy and a3 straight
+// into the LDS tile; from there the input gradient
+//   dz2[p][ci] = bf16( (sum_{k', co} Wt[ci][k'*64 + co] dz3[p + k' - 2][co]) (1 - a2[p][ci]^2) )
+// with Wt[ci][k'*64 + co] = W3[co][(4 - k')*64 + ci] (flipped, transposed), and
+// the weight gradient
+//   part[oW3 + co*320 + k*64 + ci] = sum_{rows, p} dz3[p][co] a2[p + k - 2][ci];
+// the output layer's, part[oW4 + k*64 + ci] = sum dy[p - k + 2] a3[p][ci], is
+// taken by the matrix units before dz3 replaces a3 in the tile (record tile R:
+// row p holds dy[p - k + 2], k < 5).
+// k_bwd_in: layer 2 the same way from dz2 and a1; its dz1 stays in LDS for
+// the first layer's gradient.
+//
+// Both products of a layer read the same two position-major tiles: the input
+// gradient takes the channels of a position as K (16-byte reads), the weight
+// gradient the positions (transposing reads), so a tap is a shift of the row
+// and needs no realignment.  Wave w takes output channels 16 (w & 3).. over
+// half w >> 2 of the positions for the input gradient, and input channels
+// 16 (w & 3).. by half w >> 2 of the output channels for the weight gradient.
+// The next row's tiles are loaded into registers while this row is worked on.
+// Apart (output layer, weight gradient and input gradient of each layer, first
+// layer: six kernels that passed dz1..dz3 through memory and read every
+// operand once per product) they took 917 us at 4096 rows; these two take 153
+// and 114, for 0.67 GB (140 us at the rate of a copy) and 172 GFLOP (140 us).
+// The matrix units are busy 0.2-0.3 of the time and LDS 0.3-0.5: what is left
+// is the phases between barriers, one workgroup per CU.
 // ----------------------------------------------------------------------------
-constexpr int kBwdLds = kRowsP * kP * 2;
+constexpr int kBT = 512;
+constexpr int kTile = kRowsP * kP;  // BF16 values of a tile
+constexpr int kBwdOutLds = 2 * kTile * 2 + (kRowsP + 4 + kKS * kCH) * 4 + kNV * 16 * 2;
+constexpr int kBwdInLds = 2 * kTile * 2 + kNV * 16 * 2;
 
-__global__ __launch_bounds__(256) void k_bwd_data(const bf16* dz, const bf16* wt, const bf16* ap, bf16* dzp,
-                                                   int rows) {
-  extern __shared__ __align__(16) unsigned char lds[];
-  bf16* P = reinterpret_cast<bf16*>(lds);
-  zero_pad_p(P);
-  bf16x8 A[10];
-  load_a(wt, A);
-  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
-    const size_t ro = (size_t)row * kCH * kNV;
-    stage_p(P, dz + ro);
-    __syncthreads();
-    mconv(P, A, [&](floatx4* acc, int ci0, int m) {
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+
+// MFMA operand with K = 32 rows from `row` of a tile and the 16 columns from
+// `col`: ds_read_b64_tr_b16 hands lane i of a group of 16 column i of the 4 x 16
+// block whose row r the lanes 4r..4r+3 address.  Group g takes rows 4g.. and
+// 16 + 4g.. for its 8 values of K (any order of the positions serves, both
+// operands have the same): the 8 rows that half a wave reads then lie in
+// different banks, rows 8g.. and 8g + 4.. meet two by two
+__device__ __forceinline__ bf16x8 read_rows(const bf16* tile, int pitch, int row, int col) {
+  const int l = threadIdx.x & 63;
+  const bf16* p = tile + (row + (l >> 2)) * pitch + col + 4 * (l & 3);
+  const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(__attribute__((address_space(3))) void*)p);
+  const bf16x4 hi =
+      __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(__attribute__((address_space(3))) void*)(p + 16 * pitch));
+  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// fragments of weights [64][320] for output channels 16 mt .. 16 mt + 15
+__device__ __forceinline__ void load_a_tile(const bf16* W, int mt, bf16x8 (&A)[10]) {
+  const int lane = threadIdx.x & 63;
+  const bf16* wr = W + (16 * mt + (lane & 15)) * kK + 8 * (lane >> 4);
 #pragma unroll
-      for (int nt = 0; nt < 16; ++nt) {
-        const int pos = 16 * nt + m;
+  for (int c = 0; c < 10; ++c) A[c] = *reinterpret_cast<const bf16x8*>(wr + 32 * c);
+}
+
+// a stored row [256][64] <-> registers, 16 bytes per thread and pass
+__device__ __forceinline__ void load_row(const bf16* src, bf16x8 (&v)[4]) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const bf16x8*>(src + 8 * (threadIdx.x + kBT * u));
+}
+__device__ __forceinline__ bf16* tile_at(bf16* P, int u) {
+  const int i = threadIdx.x + kBT * u;
+  return P + ((i >> 3) + 2) * kP + 8 * (i & 7);
+}
+
+// input gradient of a layer, this wave's channels and positions: dz P
+// (A: the flipped weights), a X; out[nt] = bf16(acc (1 - a^2)) of channels
+// 16 mt + 4g.. at position 16 (8 h + nt) + m
+__device__ __forceinline__ void layer_data(const bf16* P, const bf16* X, const bf16x8 (&A)[10], int mt, int h,
+                                           bf16x4 (&out)[8]) {
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  floatx4 acc[8];
+#pragma unroll
+  for (int nt = 0; nt < 8; ++nt) acc[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 10; ++c) {
+    const bf16* in = P + (128 * h + m + (c >> 1)) * kP + (c & 1) * 32 + 8 * g;
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) acc[nt] = mfma(A[c], *reinterpret_cast<const bf16x8*>(in + 16 * nt * kP), acc[nt]);
+  }
+#pragma unroll
+  for (int nt = 0; nt < 8; ++nt) {
+    const bf16x4 a = *reinterpret_cast<const bf16x4*>(X + (128 * h + 16 * nt + m + 2) * kP + 16 * mt + 4 * g);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float av = (float)a[j];
+      out[nt][j] = (bf16)(acc[nt][j] * (1.f - av * av));
+    }
+  }
+}
+
+// weight gradient of a layer, this wave's share: acc[i][k] += dz a^T for output
+// channels 16 (2 h + i).. and input channels 16 ct.., tap k; accb[i] the sums
+// of dz (kept by the waves of ct = 0)
+__device__ __forceinline__ void layer_weights(const bf16* P, const bf16* X, int ct, int h, floatx4 (&acc)[2][kKS],
+                                              floatx4 (&accb)[2]) {
+  bf16x8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ones[j] = (bf16)1.f;
+#pragma unroll 2
+  for (int c = 0; c < 8; ++c) {
+    const int p0 = 32 * c;
+    bf16x8 A[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) A[i] = read_rows(P, kP, p0 + 2, 16 * (2 * h + i));
+#pragma unroll
+    for (int k = 0; k < kKS; ++k) {
+      const bf16x8 B = read_rows(X, kP, p0 + k, 16 * ct);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i][k] = mfma(A[i], B, acc[i][k]);
+    }
+    if (ct == 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) accb[i] = mfma(A[i], ones, accb[i]);
+    }
+  }
+}
+
+__device__ __forceinline__ void write_weights(float* out, int oW, int oB, int ct, int h, const floatx4 (&acc)[2][kKS],
+                                              const floatx4 (&accb)[2]) {
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int co = 16 * (2 * h + i) + 4 * g + j;
+#pragma unroll
+      for (int k = 0; k < kKS; ++k) out[oW + co * kK + k * kCH + 16 * ct + m] = acc[i][k][j];
+      if (ct == 0 && m == 0) out[oB + co] = accb[i][j];
+    }
+  }
+}
+
+__global__ __launch_bounds__(kBT) void k_bwd_out(const float* dy, const bf16* a3, const bf16* a2, const float* p,
+                                                 const bf16* w3t, bf16* dz2, int rows, float* part) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  bf16* P = reinterpret_cast<bf16*>(lds);  // dz3
+  bf16* X = P + kTile;                     // a2
+  float* ds = reinterpret_cast<float*>(X + kTile);  // bf(dy) at p + 2
+  float* w4 = ds + kRowsP + 4;                      // bf(W4) [k][ci]
+  bf16* R = reinterpret_cast<bf16*>(w4 + kK);       // [256][16]: bf(dy[p - k + 2]), k < 5
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, m = lane & 15, g = lane >> 4;
+  const int ct = wave & 3, h = wave >> 2;
+  zero_pad_p(P);
+  zero_pad_p(X);
+  if (t < 4) ds[t < 2 ? t : kNV + t] = 0.f;
+  for (int i = t; i < kK; i += kBT) w4[i] = bfr(p[oW4 + i]);
+  for (int i = t; i < kNV * 16; i += kBT) R[i] = (bf16)0.f;
+  bf16x8 A[10];
+  load_a_tile(w3t, ct, A);
+  floatx4 acc[2][kKS], accb[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    accb[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kKS; ++k) acc[i][k] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  floatx4 acc4 = floatx4{0.f, 0.f, 0.f, 0.f};  // output layer: channels 16 ct.., half h of the positions
+  float gb = 0.f;
+  bf16x8 n3[4], n2[4];
+  float nd = 0.f;
+  auto fetch = [&](int row) {
+    const size_t ra = (size_t)row * kCH * kNV;
+    load_row(a3 + ra, n3);
+    load_row(a2 + ra, n2);
+    if (t < kNV) nd = dy[(size_t)row * kNV + t];
+  };
+  fetch(blockIdx.x);
+  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
+    bf16x8 v3[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      v3[u] = n3[u];
+      *reinterpret_cast<bf16x8*>(tile_at(P, u)) = n3[u];
+      *reinterpret_cast<bf16x8*>(tile_at(X, u)) = n2[u];
+    }
+    if (t < kNV) {
+      ds[t + 2] = bfr(nd);
+#pragma unroll
+      for (int k = 0; k < kKS; ++k) {
+        const int q = t - 2 + k;
+        if (q >= 0 && q < kNV) R[q * 16 + k] = (bf16)nd;
+      }
+      gb += nd;
+    }
+    if (row + gridDim.x < rows) fetch(row + gridDim.x);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      acc4 = mfma(read_rows(P, kP, 128 * h + 32 * c + 2, 16 * ct), read_rows(R, 16, 128 * h + 32 * c, 0), acc4);
+    // four channels at a time: with the weights of all eight the kernel spills
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      floatx4 wk[kKS];
+#pragma unroll
+      for (int k = 0; k < kKS; ++k) wk[k] = *reinterpret_cast<const floatx4*>(w4 + k * kCH + 8 * (t & 7) + 4 * q);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int pos = (t + kBT * u) >> 3;
+        float d[kKS];
+#pragma unroll
+        for (int k = 0; k < kKS; ++k) d[k] = ds[pos - k + 4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const size_t i = ro + (size_t)(ci0 + j) * kNV + pos;
-          const float av = (float)ap[i];
-          dzp[i] = (bf16)(acc[nt][j] * (1.f - av * av));
+          float s = 0.f;
+#pragma unroll
+          for (int k = 0; k < kKS; ++k) s = fmaf(wk[k][j], d[k], s);
+          const float av = (float)v3[u][4 * q + j];
+          v3[u][4 * q + j] = (bf16)(s * (1.f - av * av));
         }
       }
-    });
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // a3 read before dz3 takes its place
+#pragma unroll
+    for (int u = 0; u < 4; ++u) *reinterpret_cast<bf16x8*>(tile_at(P, u)) = v3[u];
     __syncthreads();
+    bf16x4 out[8];
+    layer_data(P, X, A, ct, h, out);
+    bf16* dst = dz2 + (size_t)row * kCH * kNV + (128 * h + m) * kCH + 16 * ct + 4 * g;
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) *reinterpret_cast<bf16x4*>(dst + 16 * nt * kCH) = out[nt];
+    layer_weights(P, X, ct, h, acc, accb);
+    __syncthreads();  // tiles read before the next row overwrites them
   }
-}
-
-// ----------------------------------------------------------------------------
-// weight gradient of a 64 -> 64 layer on MFMA (rows strided over the grid):
-//   part[wg][oW + co*320 + k*64 + ci] = sum_{rows, p} dz[co][p] x[ci][p + k - 2]
-//   part[wg][oB + co]                 = sum_{rows, p} dz[co][p]
-// GEMM M = co, N = k*64 + ci (20 tiles of 16), K = positions (8 chunks of 32).
-// ----------------------------------------------------------------------------
-constexpr int kWgtLds = 2 * kCH * kQ * 2;
-
-// 8 consecutive BF16 of an LDS row starting at element base + tap (base a
-// multiple of 8, tap in [0, 4]): two aligned 16-byte reads and a byte shift
-template <int TAP>
-__device__ __forceinline__ bf16x8 load_shift(const bf16* row, int base) {
-  const uint4 lo = *reinterpret_cast<const uint4*>(row + base);
-  if constexpr (TAP == 0) {
-    return *reinterpret_cast<const bf16x8*>(&lo);
-  } else {
-    const uint4 hi = *reinterpret_cast<const uint4*>(row + base + 8);
-    const unsigned w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    unsigned r[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if constexpr ((TAP & 1) == 0) {
-        r[q] = w[TAP / 2 + q];
-      } else {
-        r[q] = __builtin_amdgcn_alignbyte(w[(TAP + 1) / 2 + q], w[(TAP - 1) / 2 + q], 2);
-      }
-    }
-    bf16x8 out;
-    __builtin_memcpy(&out, r, 16);
-    return out;
-  }
-}
-
-__global__ __launch_bounds__(256) void k_wgrad(const bf16* dz, const bf16* x, int rows, float* part, int oW, int oB) {
-  extern __shared__ __align__(16) unsigned char lds[];
-  bf16* D = reinterpret_cast<bf16*>(lds);   // [64][kQ], element p at c*kQ + p
-  bf16* X = D + kCH * kQ;                   // [64][kQ], element p at c*kQ + p + 2
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int m = lane & 15, g = lane >> 4;
-  for (int i = t; i < kCH * (kQ - kNV); i += 256) {
-    const int c = i / (kQ - kNV), r = i % (kQ - kNV);
-    D[c * kQ + kNV + r] = (bf16)0.f;
-    const int xr = r < 2 ? r : kNV + r;  // X padding: 0, 1 and 258 .. kQ-1
-    X[c * kQ + xr] = (bf16)0.f;
-  }
-  floatx4 acc[20];
-#pragma unroll
-  for (int nt = 0; nt < 20; ++nt) acc[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float db = 0.f;
-  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
-    const size_t ro = (size_t)row * kCH * kNV;
-    // stage: 16 KB of each operand, 8 BF16 per thread per pass
-    for (int i = t; i < kCH * kNV / 8; i += 256) {
-      const int c = i / (kNV / 8), p = (i % (kNV / 8)) * 8;
-      const bf16x8 dv = *reinterpret_cast<const bf16x8*>(dz + ro + c * kNV + p);
-      const bf16x8 xv = *reinterpret_cast<const bf16x8*>(x + ro + c * kNV + p);
-      *reinterpret_cast<bf16x8*>(D + c * kQ + p) = dv;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) X[c * kQ + p + 2 + j] = xv[j];
-    }
-    __syncthreads();
-    // bias: thread t sums channel t/4 over a quarter of the positions
-    {
-      const int c = t >> 2, q = t & 3;
-      float s = 0.f;
-      for (int p = q * 64; p < q * 64 + 64; ++p) s += (float)D[c * kQ + p];
-      db += s;
-    }
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int base = 32 * c + 8 * g;
-      const bf16x8 A = *reinterpret_cast<const bf16x8*>(D + (16 * wave + m) * kQ + base);
-#pragma unroll
-      for (int nt = 0; nt < 20; ++nt) {
-        const int tap = nt >> 2;
-        const bf16* xr = X + (16 * (nt & 3) + m) * kQ;
-        bf16x8 B;
-        switch (tap) {
-          case 0: B = load_shift<0>(xr, base); break;
-          case 1: B = load_shift<1>(xr, base); break;
-          case 2: B = load_shift<2>(xr, base); break;
-          case 3: B = load_shift<3>(xr, base); break;
-          default: B = load_shift<4>(xr, base); break;
-        }
-        acc[nt] = mfma(A, B, acc[nt]);
-      }
-    }
-    __syncthreads();
-  }
-  float* out = part + (size_t)blockIdx.x * kParams;
-#pragma unroll
-  for (int nt = 0; nt < 20; ++nt) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) out[oW + (16 * wave + 4 * g + j) * kK + 16 * nt + m] = acc[nt][j];
-  }
-  db += __shfl_xor(db, 1, 64);
-  db += __shfl_xor(db, 2, 64);
-  if ((t & 3) == 0) out[oB + (t >> 2)] = db;
-}
-
-// ----------------------------------------------------------------------------
-// output layer backward (64 -> 1):
-//   dz3[ci][p] = bf16( (sum_k W4[k*64 + ci] bf(dy[p - k + 2])) (1 - a3[ci][p]^2) )
-//   part[oW4 + k*64 + ci] = sum bf(dy[p]) a3[ci][p + k - 2],  part[oB4] = sum dy
-// ----------------------------------------------------------------------------
-constexpr int kOutLds = kCH * kQs * 2 + kRowsP * 4 + 64;
-
-__global__ __launch_bounds__(256) void k_out_bwd(const float* dy, const bf16* a3, const float* p, bf16* dz3,
-                                                 int rows, float* part) {
-  extern __shared__ __align__(16) unsigned char lds[];
-  bf16* X = reinterpret_cast<bf16*>(lds);                    // a3 [64][kQs] at p + 2
-  float* ds = reinterpret_cast<float*>(lds + kCH * kQs * 2);  // bf(dy) at p + 2
-  const int t = threadIdx.x;
-  for (int i = t; i < kCH * 4; i += 256) {
-    const int c = i >> 2, r = i & 3;
-    X[c * kQs + (r < 2 ? r : kNV + r)] = (bf16)0.f;
-  }
-  if (t < 4) ds[t < 2 ? t : kNV + t] = 0.f;
-  float gw[2] = {0.f, 0.f};  // outputs o = t and o = t + 256 (o < 320)
-  float gb = 0.f;
-  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
-    const size_t ro = (size_t)row * kNV;
-    const size_t ra = (size_t)row * kCH * kNV;
-    const float d = bfr(dy[ro + t]);
-    ds[t + 2] = d;
-    gb += dy[ro + t];
-    for (int c = 0; c < kCH; ++c) X[c * kQs + t + 2] = a3[ra + (size_t)c * kNV + t];
-    __syncthreads();
-    // input gradient, thread = position
-    for (int ci = 0; ci < kCH; ++ci) {
-      float s = 0.f;
-#pragma unroll
-      for (int k = 0; k < kKS; ++k) s = fmaf(bfr(p[oW4 + k * kCH + ci]), ds[t - k + 4], s);
-      const float av = (float)X[ci * kQs + t + 2];
-      dz3[ra + (size_t)ci * kNV + t] = (bf16)(s * (1.f - av * av));
-    }
-    // weight gradient, thread = output
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int o = t + 256 * h;
-      if (o < kK) {
-        const int k = o / kCH, ci = o % kCH;
-        const bf16* xr = X + ci * kQs + k;
-        float s = 0.f;
-        for (int q = 0; q < kNV; ++q) s = fmaf(ds[q + 2], (float)xr[q], s);
-        gw[h] += s;
-      }
-    }
-    __syncthreads();
-  }
-  float* out = part + (size_t)blockIdx.x * kParams;
-  out[oW4 + t] = gw[0];
-  if (t + 256 < kK) out[oW4 + t + 256] = gw[1];
-  // bias: block sum of gb
+  float* out = part + (size_t)blockIdx.x * kPart;
+  write_weights(out, oW3, oB3, ct, h, acc, accb);
+  // output layer: the two halves of the positions
+  float* red = reinterpret_cast<float*>(lds);
+  float* redb = red + 4 * 64 * 4;
   float s = gb;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  __shared__ float red[4];
-  if ((t & 63) == 0) red[t >> 6] = s;
+  if (lane == 0) redb[wave] = s;
+  if (h == 1) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) red[(ct * 64 + lane) * 4 + j] = acc4[j];
+  }
   __syncthreads();
-  if (t == 0) out[oB4] = (red[0] + red[1]) + (red[2] + red[3]);
+  if (h == 0 && m < kKS) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[oW4 + m * kCH + 16 * ct + 4 * g + j] = acc4[j] + red[(ct * 64 + lane) * 4 + j];
+  }
+  if (t == 0) out[oB4] = (redb[0] + redb[1]) + (redb[2] + redb[3]);
 }
 
-// ----------------------------------------------------------------------------
-// first layer weight gradient (1 -> 64):
-//   part[oW1 + c*5 + k] = sum dz1[c][p] x[p + k - 2],  part[oB1 + c] = sum dz1[c][p]
-// ----------------------------------------------------------------------------
-constexpr int kInLds = kCH * kQs * 2 + kRowsP * 4 + 64;
-
-__global__ __launch_bounds__(256) void k_in_wgrad(const bf16* dz1, const bf16* xin, int rows, float* part) {
+// first layer (1 -> 64), from dz1 in P: part[oW1 + c*5 + k] = sum dz1[p][c]
+// x[p + k - 2], part[oB1 + c] = sum dz1[p][c], as one product with the record
+// tile R [256][16] whose row p holds x[p-2..p+2], 1 and zeros
+__global__ __launch_bounds__(kBT) void k_bwd_in(const bf16* dz2, const bf16* a1, const bf16* xin, const bf16* w2t,
+                                                int rows, float* part) {
   extern __shared__ __align__(16) unsigned char lds[];
-  bf16* D = reinterpret_cast<bf16*>(lds);                     // dz1 [64][kQs]
-  float* xs = reinterpret_cast<float*>(lds + kCH * kQs * 2);  // x at p + 2
-  const int t = threadIdx.x;
-  if (t < 4) xs[t < 2 ? t : kNV + t] = 0.f;
-  // thread t: channel c = t / 4, outputs (k = 0..4, bias) over positions q*64 .. q*64+63
-  const int c = t >> 2, q = t & 3;
-  float gw[kKS + 1] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
-    const size_t ra = (size_t)row * kCH * kNV;
-    xs[t + 2] = (float)xin[(size_t)row * kNV + t];
-    for (int cc = 0; cc < kCH; ++cc) D[cc * kQs + t] = dz1[ra + (size_t)cc * kNV + t];
-    __syncthreads();
-    for (int pp = q * 64; pp < q * 64 + 64; ++pp) {
-      const float dv = (float)D[c * kQs + pp];
+  bf16* P = reinterpret_cast<bf16*>(lds);  // dz2, then dz1
+  bf16* X = P + kTile;                     // a1
+  bf16* R = X + kTile;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, m = lane & 15, g = lane >> 4;
+  const int ct = wave & 3, h = wave >> 2;
+  zero_pad_p(P);
+  zero_pad_p(X);
+  for (int i = t; i < kNV * 16; i += kBT) R[i] = (bf16)((i & 15) == kKS ? 1.f : 0.f);
+  bf16x8 A[10];
+  load_a_tile(w2t, ct, A);
+  floatx4 acc[2][kKS], accb[2], acc1 = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int k = 0; k < kKS; ++k) gw[k] = fmaf(dv, xs[pp + k], gw[k]);
-      gw[kKS] += dv;
+  for (int i = 0; i < 2; ++i) {
+    accb[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kKS; ++k) acc[i][k] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  bf16x8 nz[4], na[4];
+  bf16 nxv = (bf16)0.f;
+  auto fetch = [&](int row) {
+    const size_t ra = (size_t)row * kCH * kNV;
+    load_row(dz2 + ra, nz);
+    load_row(a1 + ra, na);
+    if (t < kNV) nxv = xin[(size_t)row * kNV + t];
+  };
+  fetch(blockIdx.x);
+  __syncthreads();  // R cleared before any thread writes a record
+  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      *reinterpret_cast<bf16x8*>(tile_at(P, u)) = nz[u];
+      *reinterpret_cast<bf16x8*>(tile_at(X, u)) = na[u];
+    }
+    if (t < kNV) {
+#pragma unroll
+      for (int k = 0; k < kKS; ++k) {
+        const int q = t + 2 - k;
+        if (q >= 0 && q < kNV) R[q * 16 + k] = nxv;
+      }
+    }
+    if (row + gridDim.x < rows) fetch(row + gridDim.x);
+    __syncthreads();
+    bf16x4 out[8];
+    layer_data(P, X, A, ct, h, out);
+    layer_weights(P, X, ct, h, acc, accb);
+    __syncthreads();  // dz2 read before dz1 takes its place
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt)
+      *reinterpret_cast<bf16x4*>(P + (128 * h + 16 * nt + m + 2) * kP + 16 * ct + 4 * g) = out[nt];
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int p0 = 128 * h + 32 * c;
+      acc1 = mfma(read_rows(P, kP, p0 + 2, 16 * ct), read_rows(R, 16, p0, 0), acc1);
     }
     __syncthreads();
   }
+  float* out = part + (size_t)blockIdx.x * kPart;
+  write_weights(out, oW2, oB2, ct, h, acc, accb);
+  // the two halves of the positions
+  float* red = reinterpret_cast<float*>(lds);
+  if (h == 1) {
 #pragma unroll
-  for (int k = 0; k <= kKS; ++k) {
-    gw[k] += __shfl_xor(gw[k], 1, 64);
-    gw[k] += __shfl_xor(gw[k], 2, 64);
+    for (int j = 0; j < 4; ++j) red[(ct * 64 + lane) * 4 + j] = acc1[j];
   }
-  if (q == 0) {
-    float* out = part + (size_t)blockIdx.x * kParams;
+  __syncthreads();
+  if (h == 0) {
 #pragma unroll
-    for (int k = 0; k < kKS; ++k) out[oW1 + c * kKS + k] = gw[k];
-    out[oB1 + c] = gw[kKS];
+    for (int j = 0; j < 4; ++j) {
+      const float s = acc1[j] + red[(ct * 64 + lane) * 4 + j];
+      const int c = 16 * ct + 4 * g + j;
+      if (m < kKS) out[oW1 + c * kKS + m] = s;
+      if (m == kKS) out[oB1 + c] = s;
+    }
   }
 }
 
-// grad[i] = sum over workgroups of part[wg][i]; loss = sum of loss_rows * lscale
-__global__ __launch_bounds__(256) void k_reduce(const float* part, int nwg, float* grad, const float* loss_rows,
-                                                int rows, float lscale, float* loss) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < kParams) {
+// grad[i] = sum over workgroups of part[wg][i], 256 parameters per workgroup
+// and a sixteenth of the partials per wave, 16 loads in flight; the workgroup
+// past the parameters forms loss = sum of loss_rows * lscale.  (256 partials:
+// one thread per parameter with one load at a time 99 us, with 16 loads in
+// flight 33 us, with 16-byte ones here 10.)
+constexpr int kReduceWG = (kPart + 255) / 256;
+
+__global__ __launch_bounds__(1024) void k_reduce(const float* part, int nwg, float* grad, const float* loss_rows,
+                                                 int rows, float lscale, float* loss) {
+  __shared__ floatx4 red[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (blockIdx.x == kReduceWG) {
     float s = 0.f;
-    for (int w = 0; w < nwg; ++w) s += part[(size_t)w * kParams + i];
-    grad[i] = s;
-  }
-  if (blockIdx.x == 0 && loss) {
-    __shared__ float red[4];
-    float s = 0.f;
-    for (int r = threadIdx.x; r < rows; r += 256) s += loss_rows[r];
+    for (int r = threadIdx.x; r < rows; r += 1024) s += loss_rows[r];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    float* rs = reinterpret_cast<float*>(red);
+    if (lane == 0) rs[wave] = s;
     __syncthreads();
-    if (threadIdx.x == 0) *loss = ((red[0] + red[1]) + (red[2] + red[3])) * lscale;
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1)
+        for (int w = 0; w < o; ++w) rs[w] += rs[w + o];
+      *loss = rs[0] * lscale;
+    }
+    return;
   }
+  const int i = 256 * blockIdx.x + 4 * lane;
+  floatx4 acc[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) acc[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (i < kPart) {
+    for (int w = wave; w < nwg; w += 256) {
+      floatx4 v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int q = w + 16 * u;
+        v[u] = *reinterpret_cast<const floatx4*>(part + (size_t)(q < nwg ? q : w) * kPart + i);
+      }
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (w + 16 * u < nwg) acc[u & 3] += v[u];
+    }
+  }
+  red[wave][lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  __syncthreads();
+  if (wave >= 4) return;
+  // parameter 256 blockIdx + threadIdx of the 16 waves' sums
+  const float* rs = reinterpret_cast<const float*>(red) + threadIdx.x;
+  float s = 0.f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) s += rs[256 * w];
+  const int j = 256 * blockIdx.x + threadIdx.x;
+  if (j < kParams) grad[j] = s;
 }
 
 // BF16 copies of W2, W3 ([co][k*64+ci]) and their flipped transposes
@@ -651,7 +777,7 @@ struct vpfc_net_s {
   float* grad = nullptr;
   float* part = nullptr;
   bf16 *w2 = nullptr, *w3 = nullptr, *w2t = nullptr, *w3t = nullptr;
-  bf16 *xin = nullptr, *a1 = nullptr, *a2 = nullptr, *a3 = nullptr, *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr;
+  bf16 *xin = nullptr, *a1 = nullptr, *a2 = nullptr, *a3 = nullptr, *dz2 = nullptr;
   float* dy = nullptr;
   float* loss_rows = nullptr;
   float* loss = nullptr;
@@ -682,8 +808,10 @@ int launched() {
 int set_lds_all() {
   static bool done = false;
   if (done) return VPFP_OK;
-  FC_HIP(hipFuncSetAttribute((const void*)k_fwd, hipFuncAttributeMaxDynamicSharedMemorySize, kFwdLds));
-  FC_HIP(hipFuncSetAttribute((const void*)k_wgrad, hipFuncAttributeMaxDynamicSharedMemorySize, kWgtLds));
+  FC_HIP(hipFuncSetAttribute((const void*)k_fwd<false>, hipFuncAttributeMaxDynamicSharedMemorySize, kFwdLds));
+  FC_HIP(hipFuncSetAttribute((const void*)k_fwd<true>, hipFuncAttributeMaxDynamicSharedMemorySize, kFwdLds));
+  FC_HIP(hipFuncSetAttribute((const void*)k_bwd_out, hipFuncAttributeMaxDynamicSharedMemorySize, kBwdOutLds));
+  FC_HIP(hipFuncSetAttribute((const void*)k_bwd_in, hipFuncAttributeMaxDynamicSharedMemorySize, kBwdInLds));
   done = true;
   return VPFP_OK;
 }
@@ -714,7 +842,10 @@ FwdArgs fwd_args(vpfc_net_t n, const float* x, int rows) {
 int run_fwd(const FwdArgs& a, hipStream_t s) {
   if (a.rows == 0) return VPFP_OK;
   if (int rc = set_lds_all()) return rc;
-  hipLaunchKernelGGL(k_fwd, dim3(fwd_grid(a.rows)), dim3(256), kFwdLds, s, a);
+  if (a.dy)
+    hipLaunchKernelGGL(k_fwd<true>, dim3(fwd_grid(a.rows)), dim3(256), kFwdLds, s, a);
+  else
+    hipLaunchKernelGGL(k_fwd<false>, dim3(fwd_grid(a.rows)), dim3(256), kFwdLds, s, a);
   return launched();
 }
 
@@ -732,20 +863,13 @@ int gradients(vpfc_net_t n, const float* x, const float* target, int rows, float
   a.dy = n->dy;
   a.loss_rows = n->loss_rows;
   if (int rc = run_fwd(a, s)) return rc;
-  const int G = kPartWG;
-  hipLaunchKernelGGL(k_out_bwd, dim3(G), dim3(256), kOutLds, s, n->dy, n->a3, n->p, n->dz3, rows, n->part);
+  const int G = rows < kPartWG ? rows : kPartWG;
+  hipLaunchKernelGGL(k_bwd_out, dim3(G), dim3(kBT), kBwdOutLds, s, n->dy, n->a3, n->a2, n->p, n->w3t, n->dz2, rows,
+                     n->part);
   if (int rc = launched()) return rc;
-  hipLaunchKernelGGL(k_wgrad, dim3(G), dim3(256), kWgtLds, s, n->dz3, n->a2, rows, n->part, oW3, oB3);
+  hipLaunchKernelGGL(k_bwd_in, dim3(G), dim3(kBT), kBwdInLds, s, n->dz2, n->a1, n->xin, n->w2t, rows, n->part);
   if (int rc = launched()) return rc;
-  hipLaunchKernelGGL(k_bwd_data, dim3(fwd_grid(rows)), dim3(256), kBwdLds, s, n->dz3, n->w3t, n->a2, n->dz2, rows);
-  if (int rc = launched()) return rc;
-  hipLaunchKernelGGL(k_wgrad, dim3(G), dim3(256), kWgtLds, s, n->dz2, n->a1, rows, n->part, oW2, oB2);
-  if (int rc = launched()) return rc;
-  hipLaunchKernelGGL(k_bwd_data, dim3(fwd_grid(rows)), dim3(256), kBwdLds, s, n->dz2, n->w2t, n->a1, n->dz1, rows);
-  if (int rc = launched()) return rc;
-  hipLaunchKernelGGL(k_in_wgrad, dim3(G), dim3(256), kInLds, s, n->dz1, n->xin, rows, n->part);
-  if (int rc = launched()) return rc;
-  hipLaunchKernelGGL(k_reduce, dim3((kParams + 255) / 256), dim3(256), 0, s, n->part, G, grad, n->loss_rows, rows,
+  hipLaunchKernelGGL(k_reduce, dim3(kReduceWG + (loss ? 1 : 0)), dim3(1024), 0, s, n->part, G, grad, n->loss_rows, rows,
                      1.f / count, loss);
   return launched();
 }
@@ -768,7 +892,7 @@ int vpfc_create(int max_rows, vpfc_net_t* out) {
   if (!rc) rc = nalloc(n, &n->mo, sizeof(float) * kParams);
   if (!rc) rc = nalloc(n, &n->ve, sizeof(float) * kParams);
   if (!rc) rc = nalloc(n, &n->grad, sizeof(float) * kParams);
-  if (!rc) rc = nalloc(n, &n->part, sizeof(float) * kParams * kPartWG);
+  if (!rc) rc = nalloc(n, &n->part, sizeof(float) * kPart * kPartWG);
   if (!rc) rc = nalloc(n, &n->w2, sizeof(bf16) * kCH * kK);
   if (!rc) rc = nalloc(n, &n->w3, sizeof(bf16) * kCH * kK);
   if (!rc) rc = nalloc(n, &n->w2t, sizeof(bf16) * kCH * kK);
@@ -777,9 +901,7 @@ int vpfc_create(int max_rows, vpfc_net_t* out) {
   if (!rc) rc = nalloc(n, &n->a1, act);
   if (!rc) rc = nalloc(n, &n->a2, act);
   if (!rc) rc = nalloc(n, &n->a3, act);
-  if (!rc) rc = nalloc(n, &n->dz1, act);
   if (!rc) rc = nalloc(n, &n->dz2, act);
-  if (!rc) rc = nalloc(n, &n->dz3, act);
   if (!rc) rc = nalloc(n, &n->dy, R * kNV * sizeof(float));
   if (!rc) rc = nalloc(n, &n->loss_rows, R * sizeof(float));
   if (!rc) rc = nalloc(n, &n->loss, sizeof(float));
