@@ -729,7 +729,7 @@ VP_HD void row_sum(Ctx& c, double* vals, double* scratch) {
 // return `d` holds the solution.  Coef::view<L>(m0, first, last) gives the
 // thread's coefficients l(i), u(i), b(i) of row m0 + i (zero l(0) on the
 // first thread and u(L-1) on the last).
-// red: 5*TPT doubles of LDS for the interface system (one row per thread
+// red: 8*TPT doubles of LDS for the interface system (one row per thread
 // after the even interface unknowns are eliminated).
 // ---------------------------------------------------------------------------
 // FULL: reciprocals to full double precision (FP64 f); otherwise to ~2^-46
@@ -783,26 +783,52 @@ VP_HD void tridiag(Ctx& c, double* d, const Coef& cf, int t, double* red) {
   // first).  It is a Schur complement of the diagonally dominant system,
   // hence diagonally dominant itself, and is solved by parallel cyclic
   // reduction, one row per thread.
-  double* A = red;
-  double* B = red + TPT;
-  double* C = red + 2 * TPT;
-  double* D = red + 3 * TPT;
-  A[t] = p2;
-  B[t] = q2;
-  C[t] = r2;
+  //
+  // A level whose update changes no row's B or D (the couplings have fallen
+  // below the rounding of the rows they reach) ends the reduction: those of the
+  // levels after it are the squares.  Weak collisions (nu dt T/dv^2 ~ 1, 16 rows
+  // per chunk) need 3-4 of 7 levels, strong ones all.  Two buffers take turns,
+  // so a level has one barrier.  With two
+  // barriers and every level: 64 x 1024 FP64 step 18.2 us, with this 17.9;
+  // 1024 x 8192 FP64 row launch 120 -> 115 us, FP32 92.5 -> 87.5.
+  constexpr int NW = TPT > 64 ? TPT / 64 : 1;
+  unsigned* vote = reinterpret_cast<unsigned*>(red + 8 * TPT);  // [2][NW], TPT > 64 only
+  double* X = red + 4 * TPT;
+  X[t] = p2;
+  X[TPT + t] = q2;
+  X[2 * TPT + t] = r2;
   c.sync();
   const bool last = t == TPT - 1;
-  const double p2n = last ? 0.0 : A[t + 1], q2n = last ? 0.0 : B[t + 1], r2n = last ? 0.0 : C[t + 1];
-  c.sync();
+  const double p2n = last ? 0.0 : X[t + 1], q2n = last ? 0.0 : X[TPT + t + 1], r2n = last ? 0.0 : X[2 * TPT + t + 1];
   double ra = q * r2, rb = 1.0 - q * q2 - r * r2n, rc = r * q2n, rd = p + q * p2 - r * p2n;
   // each thread publishes 1/B of its row with it (one reciprocal per level)
-  double* BI = red + 4 * TPT;
+  double bi = rcpp<FULL>(rb);
+  bool changed = true;
+  int o = 0;  // buffer of this level
   for (int s = 1; s < TPT; s <<= 1) {
+    if constexpr (TPT <= 64) {
+      if (!c.any(changed)) break;
+    }
+    double* A = red + o;
+    double* BI = A + TPT;
+    double* C = A + 2 * TPT;
+    double* D = A + 3 * TPT;
     A[t] = ra;
-    BI[t] = rcpp<FULL>(rb);
+    BI[t] = bi;
     C[t] = rc;
     D[t] = rd;
-    c.sync();
+    if constexpr (TPT > 64) {
+      unsigned* vw = vote + (o ? NW : 0);
+      const bool w = c.any(changed);
+      if ((t & 63) == 0) vw[t >> 6] = w;
+      c.sync();
+      unsigned go = 0;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) go |= vw[i];
+      if (!go) break;
+    } else {
+      c.sync();
+    }
     const int im = t - s, ip = t + s;
     double na = 0.0, nb = rb, nc = 0.0, nd = rd;
     if (im >= 0) {
@@ -817,17 +843,20 @@ VP_HD void tridiag(Ctx& c, double* d, const Coef& cf, int t, double* red) {
       nb += ga * A[ip];
       nd += ga * D[ip];
     }
+    changed = !(nb == rb && nd == rd);  // true for NaN: it spreads as it does without the test
     ra = na;
     rb = nb;
     rc = nc;
     rd = nd;
-    c.sync();
+    bi = rcpp<FULL>(rb);
+    o = 4 * TPT - o;
   }
-  const double xe = rd * rcpp<FULL>(rb);
+  const double xe = rd * bi;
   // y_{2t} = p2 - r2 z_{t-1} + q2 z_t
-  A[t] = xe;
+  X = red + o;  // not read by any thread still in the last level
+  X[t] = xe;
   c.sync();
-  const double zm = t > 0 ? A[t - 1] : 0.0;
+  const double zm = t > 0 ? X[t - 1] : 0.0;
   c.sync();
   const double xs = p2 - r2 * zm + q2 * xe;
   // interior rows with both chunk ends known

@@ -390,7 +390,7 @@ struct RowCfg {
   static constexpr int TPT = M / Q;
   static constexpr int L = 2 * Q;
   static constexpr int fft_bytes = Padded<M>::size * (int)sizeof(cx<T>);
-  static constexpr int red_bytes = 8 * TPT * 8;
+  static constexpr int red_bytes = 8 * TPT * 8 + (TPT > 64 ? TPT / 64 * 8 : 0);
   static constexpr int region = ((fft_bytes > red_bytes ? fft_bytes : red_bytes) + 15) & ~15;
   static constexpr int wg = TPT >= 64 ? TPT : 64;
   static constexpr int rows = wg / TPT;
@@ -400,10 +400,12 @@ struct RowCfg {
   static constexpr int pro_bytes = ProCfg<wg>::bytes;
   static constexpr int main_bytes = rows * region + sum_bytes;
   static constexpr int lds = main_bytes > pro_bytes ? main_bytes : pro_bytes;
-  // minimum waves per SIMD asked of the register allocator: 3 (168 VGPRs,
-  // small spills) measured faster than 2 for FP32 rows with M <= 1024 (the
-  // scan's classes) and slower for FP64 and for M = 4096
-  static constexpr int min_waves = (Q == 8 && sizeof(T) == 4 && M <= 1024) ? 3 : 1;
+  // minimum waves per SIMD asked of the register allocator: 3 (168 VGPRs) for
+  // 8 values per thread and M <= 1024, the scans' classes, which otherwise come
+  // out at 170 now and then and run two waves (FP64 M = 1024, 512 instances: 153
+  // against 174 us); 4 spills 100 to 260 bytes and is slower (FP32 delta-f
+  // M = 1024, 4096 instances 1116 -> 1431 us; M = 4096 FP64, 1024 rows 115 -> 134)
+  static constexpr int min_waves = (Q == 8 && M <= 1024) ? 3 : 1;
 };
 
 // BG: delta-f storage (a.bg, a.bg_hat set); a kernel of its own so that the

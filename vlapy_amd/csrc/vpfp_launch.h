@@ -31,6 +31,7 @@ struct GpuCtx {
   }
   __device__ __forceinline__ double shfl_xor(double v, int m, int w) { return __shfl_xor(v, m, w); }
   __device__ __forceinline__ float shfl_xor(float v, int m, int w) { return __shfl_xor(v, m, w); }
+  __device__ __forceinline__ bool any(bool p) { return __any(p); }
   // v of the lane opposite in bit MASK: a DPP move for MASK < 16 (row_mirror
   // and row_half_mirror pair lane l with 15 - l and 7 - l, which also differ
   // in the lower bits: callers only need equal higher bits)
