@@ -115,14 +115,23 @@ template <class T, int M, int Q, int C>
 __global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg)) void k_drift(vp::DriftArgs<T> a) {
   extern __shared__ __align__(16) unsigned char lds[];
   VPFP_CTX;
-  vp::drift_body<T, M, Q, C>(c, lds, a);
+  vp::drift_body<T, M, Q, C, false, unsigned long>(c, lds, a);  // any nv
+}
+
+// one column tile per workgroup (nv at most kDriftMaxWG tiles of 32)
+template <class T, int M, int Q, int C>
+__global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg), (vp::DriftCfg<T, M, Q, C>::min_waves)) void k_drift_one(
+    vp::DriftArgs<T> a) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  VPFP_CTX;
+  vp::drift_body<T, M, Q, C, true, unsigned>(c, lds, a);
 }
 
 template <class T, int M, int C>
 int launch_drift_c(const vp::DriftArgs<T>& a, hipStream_t s, int gx, int gy) {
   constexpr int Q = vp::drift_q<T>(M);
   using Cfg = vp::DriftCfg<T, M, Q, C>;
-  auto kern = k_drift<T, M, Q, C>;
+  auto kern = a.nv == gx * C ? k_drift_one<T, M, Q, C> : k_drift<T, M, Q, C>;
   if (Cfg::wg > 1024 || Cfg::lds > kMaxLds)
     return fail(VPFP_EUNSUPPORTED, "drift tile of " + std::to_string(C) + " columns does not fit a workgroup");
   if (a.fuse_field && !Cfg::tail) return fail(VPFP_EUNSUPPORTED, "field tail not available at this size");
@@ -163,7 +172,10 @@ __global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg)) void k_drift_multi(
   a.xcd_order = 0;
   a.fuse_field = 0;
   GpuCtx c{(int)threadIdx.x, (int)blockDim.x, local % gx, gx, local / gx};
-  vp::drift_body<T, M, Q, C>(c, lds, a);
+  // nv <= 8192.  64-bit offsets for the longer columns all the same (nx = 128
+  // FP32, 4096 instances: 280 us, with 32-bit ones 288; nx = 64: 124 and 114)
+  using Off = std::conditional_t<(M <= 32), unsigned, unsigned long>;
+  vp::drift_body<T, M, Q, C, false, Off>(c, lds, a);
 }
 
 template <class T, int M, int C>

@@ -43,7 +43,7 @@ VP_HD void spectral_apply(Ctx& c, cx<T>* v, cx<T>* buf, const Tw<T>& tw, int t, 
   }
   cx<T> wk[Q];
 #pragma unroll
-  for (int i = 0; i < Q; ++i) wk[i] = tw.w[t + i * TPT];
+  for (int i = 0; i < Q; ++i) wk[i] = at(tw.w + i * TPT, (unsigned)t);
   c.sync();
   cx<T> pz[Q];
 #pragma unroll
@@ -440,7 +440,7 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
   const cx<T>* src = reinterpret_cast<const cx<T>*>(a.f_in + (size_t)rowc * a.nv);
   cx<T> v[Q];
 #pragma unroll
-  for (int i = 0; i < Q; ++i) v[i] = src[t + i * TPT];
+  for (int i = 0; i < Q; ++i) v[i] = at(src + i * TPT, (unsigned)t);
   double e = 0.0;
   if (a.field_pro) {
     e = field_rows<Cfg::wg, TPT>(c, a.fld, lds, rowc, valid, t);
@@ -499,7 +499,7 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
     const int m0 = t * L;
     if constexpr (BG) {
 #pragma unroll
-      for (int i = 0; i < L; ++i) d[i] += a.bg[m0 + i];
+      for (int i = 0; i < L; ++i) d[i] += at(a.bg + i, (unsigned)m0);
     }
     const double nu_dt = a.nu_dt_inst ? a.nu_dt_inst[rowc / a.rows_per_inst] : a.nu_dt;
     if ((a.flags & RK_COLLIDE) && nu_dt > 0.0) {
@@ -567,7 +567,7 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
     }
     if constexpr (BG) {
 #pragma unroll
-      for (int i = 0; i < L; ++i) d[i] -= a.bg[m0 + i];
+      for (int i = 0; i < L; ++i) d[i] -= at(a.bg + i, (unsigned)m0);
     }
     // chunk -> natural order
 #pragma unroll
@@ -588,7 +588,7 @@ VP_HD void row_body(Ctx& c, unsigned char* lds, const RowArgs<T>& a) {
   if (valid && a.f_out) {
     cx<T>* dst = reinterpret_cast<cx<T>*>(a.f_out + (size_t)row * a.nv);
 #pragma unroll
-    for (int i = 0; i < Q; ++i) dst[t + i * TPT] = v[i];
+    for (int i = 0; i < Q; ++i) at(dst + i * TPT, (unsigned)t) = v[i];
   }
 }
 
@@ -798,9 +798,16 @@ struct DriftCfg {
   static constexpr bool tail = M <= 128 && (M / fq) <= wg;
   static constexpr int field_lds = tail ? FieldCfg<M, fq, wg>::lds : 0;
   static constexpr int lds = own > field_lds ? own : field_lds;
+  // one tile per workgroup (ONE): without the next tile's values and the running
+  // density in registers, two workgroups of eight waves fit a CU, and one loads
+  // while the other transforms (nx = 1024, nv = 8192: FP32 36.2 -> 27.3 us; FP64,
+  // which spills 88 bytes for it, 55 -> 47)
+  static constexpr int min_waves = wg == 512 && 2 * lds <= 160 * 1024 ? 4 : 1;
 };
 
-template <class T, int M, int Q, int C, class Ctx>
+// ONE: one tile per workgroup.  Off: the type of an element's offset from the
+// first row of a tile (32 bits where nx nv is known to allow it)
+template <class T, int M, int Q, int C, bool ONE, class Off, class Ctx>
 VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
   using Cfg = DriftCfg<T, M, Q, C>;
   constexpr int TPT = Cfg::TPT;
@@ -811,6 +818,7 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
   const int inst = c.bidy;
   const size_t foff = (size_t)inst * (size_t)a.nx * nv;
   const double dk = a.dk_inst ? a.dk_inst[inst] : a.dk;
+  const Off xo = (Off)(2 * t) * (Off)a.nv + (Off)cc;  // row 2t of a tile's column cc
   Tw<T> tw = tw_at<M, Q>(a.tw);
   if constexpr (Cfg::stage) {
     cx<T>* tl = reinterpret_cast<cx<T>*>(lds);
@@ -818,8 +826,6 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
     tw = Tw<T>{tl, tl + M};
   }
   double acc[2 * Q];
-#pragma unroll
-  for (int i = 0; i < 2 * Q; ++i) acc[i] = 0.0;
   const int ntiles = a.nv / C;
   // workgroup b takes the run of `per` consecutive column tiles starting at
   // b per (per = ntiles / workgroups rounded up): neighbouring narrow tiles
@@ -828,37 +834,55 @@ VP_HD void drift_body(Ctx& c, unsigned char* lds, const DriftArgs<T>& a) {
   const int b0 = a.xcd_order ? xcd_block(c.bid, c.nblk) : c.bid;
   const int per = (ntiles + c.nblk - 1) / c.nblk;
   const int t0 = b0 * per, t1 = t0 + per < ntiles ? t0 + per : ntiles;
-  // the next tile's columns are loaded before this tile's transforms, so
-  // its reads are in flight during them
-  cx<T> v[Q], nxt[Q];
-  double vc_next = 0.0;
   auto load = [&](int tile, cx<T>* dst, double& vcol) {
-    const T* fi = a.f_in + foff + tile * C + cc;
+    const T* fi = a.f_in + foff + tile * C;
 #pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      const int j = t + i * TPT;
-      dst[i] = mk<T>(fi[(size_t)(2 * j) * nv], fi[(size_t)(2 * j + 1) * nv]);
-    }
-    vcol = a.v[tile * C + cc];
+    for (int i = 0; i < Q; ++i)
+      dst[i] = mk<T>(at(fi + (size_t)(2 * i * TPT) * nv, xo), at(fi + (size_t)(2 * i * TPT + 1) * nv, xo));
+    vcol = at(a.v + tile * C, (unsigned)cc);
   };
-  if (t0 < t1) load(t0, nxt, vc_next);
-  if constexpr (Cfg::stage) c.sync();
-  for (int tile = t0; tile < t1; ++tile) {
-    const int col = tile * C + cc;
-#pragma unroll
-    for (int i = 0; i < Q; ++i) v[i] = nxt[i];
-    const double vc = vc_next;
-    if (tile + 1 < t1) load(tile + 1, nxt, vc_next);
+  auto advect = [&](int tile, cx<T>* v, double vc) {
     spectral_apply<T, M, TPT>(c, v, buf, tw, t, PhaseMul<T>((dk * a.dt) * vc, M, t, TPT));
-    T* fo = a.f_out + foff + col;
-    const double w = trapw(col, a.nv);
+    T* fo = a.f_out + foff + tile * C;
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-      const int j = t + i * TPT;
-      fo[(size_t)(2 * j) * nv] = v[i].re;
-      fo[(size_t)(2 * j + 1) * nv] = v[i].im;
-      acc[2 * i] += w * (double)v[i].re;
-      acc[2 * i + 1] += w * (double)v[i].im;
+      at(fo + (size_t)(2 * i * TPT) * nv, xo) = v[i].re;
+      at(fo + (size_t)(2 * i * TPT + 1) * nv, xo) = v[i].im;
+    }
+  };
+  cx<T> v[Q];
+  double vc = 0.0;
+  if constexpr (ONE) {
+    load(b0, v, vc);
+    if constexpr (Cfg::stage) c.sync();
+    advect(b0, v, vc);
+    const double w = trapw(b0 * C + cc, a.nv);
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+      acc[2 * i] = w * (double)v[i].re;
+      acc[2 * i + 1] = w * (double)v[i].im;
+    }
+  } else {
+    // the next tile's columns are loaded before this tile's transforms, so
+    // its reads are in flight during them
+    cx<T> nxt[Q];
+    double vc_next = 0.0;
+#pragma unroll
+    for (int i = 0; i < 2 * Q; ++i) acc[i] = 0.0;
+    if (t0 < t1) load(t0, nxt, vc_next);
+    if constexpr (Cfg::stage) c.sync();
+    for (int tile = t0; tile < t1; ++tile) {
+#pragma unroll
+      for (int i = 0; i < Q; ++i) v[i] = nxt[i];
+      vc = vc_next;
+      if (tile + 1 < t1) load(tile + 1, nxt, vc_next);
+      advect(tile, v, vc);
+      const double w = trapw(tile * C + cc, a.nv);
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        acc[2 * i] += w * (double)v[i].re;
+        acc[2 * i + 1] += w * (double)v[i].im;
+      }
     }
   }
   if (a.dens) {

@@ -63,6 +63,9 @@ __global__ __launch_bounds__((vp::RowCfg<T, M, Q>::wg), (vp::RowCfg<T, M, Q>::mi
   a.nu_dt_inst = m.seg[s].nu_dt;
   a.nx = m.seg[s].rows;
   a.rows_per_inst = m.seg[s].rows_per_inst;
+  a.field_pro = 0;  // single grids only
+  a.prev_series = nullptr;
+  a.xm_out = nullptr;
   GpuCtx c{(int)threadIdx.x, (int)blockDim.x, (int)blockIdx.x - m.seg[s].blk0, 0, 0};
   vp::row_body<T, M, Q, GpuCtx, BG>(c, lds, a);
 }
