@@ -271,8 +271,10 @@ int vpfp_batch_background(vpfp_batch_t batch, void* f, int sign, void* stream);
  * counterpart in the reference (its NumPy path has no launch shapes); the
  * choices change rounding only, never the algorithm.
  *   row_q       values per thread of the v-direction row kernels: 4
- *               (16 <= nv/2 <= 2048), 8, or 16 (nv/2 >= 256); 0 = by row
- *               count (4 when the grid has few rows, else 8)
+ *               (16 <= nv/2 <= 2048), 8, or 16 (nv/2 >= 256; with delta-f
+ *               storage only FP32 at nv = 8192, 8 run elsewhere); 0 = by row
+ *               count (4 when the grid has few rows, 16 for many FP32 rows
+ *               of nv = 8192, else 8)
  *   drift_tile  x-advection columns per workgroup: 4, 8, 16 or 32 (0 = keep)
  *   fuse_field  0: the field is a launch of its own; 1: the last drift
  *               workgroup solves it (nx <= 256); 2: every row workgroup forms

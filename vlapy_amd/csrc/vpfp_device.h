@@ -301,9 +301,15 @@ VP_HD void butterfly(cx<T>& a, cx<T>& b, int J) {
   }
   const double cd = cos32(J), sd = INV ? -sin32(J) : sin32(J);
   const bool cbig = (cd < 0 ? -cd : cd) >= (sd < 0 ? -sd : sd);
-  const T f = (T)(cbig ? cd : sd), r = (T)(cbig ? sd / cd : cd / sd);
+  // r from the rounded f so that f^2 (1 + r^2) = 1 as near as r allows: the two
+  // transforms of a pusher multiply by W and its conjugate, so an error of the
+  // angle drops out and one of the modulus scales modes, step after step (FP32
+  // rows at 16 values, whose W are not only multiples of 45 degrees)
+  const double big = cbig ? cd : sd, small = cbig ? sd : cd;
+  const T f = (T)big;
+  const T r = (T)((small + (big - (double)f) * (big + (double)f) / (2.0 * small)) / (double)f);
   // W b = (b.re c + b.im s, b.im c - b.re s)
-  const bool one = r == T(1), mone = r == T(-1);
+  const bool one = (J & 3) == 0 && r > T(0), mone = (J & 3) == 0 && r < T(0);  // odd multiples of 45 degrees
   T u, w;
   if (cbig) {
     u = one ? b.re + b.im : mone ? b.re - b.im : b.re + r * b.im;
@@ -484,11 +490,14 @@ VP_HD cx<T> half_phase(T C, T S, T s) {
 // bin instead of 44 for the three steps apart; with the last Stockham passes
 // kept in registers: nv = 8192 FP64 kicks 69 -> 63 us (1024 rows), nx = 1024
 // FP64 drift 66 -> 59 us, nx = 128 FP32 drift of a scan 503 -> 482 us.  Bins
-// are visited in the order k = t, t + TPT, ..., so p_k is a running product.
+// are visited in the order k = t, t + TPT, ..., so p_k is a running product, of
+// at most 8 factors: with 16 bins per thread it starts anew at the 9th, whose
+// rounding otherwise grows with them (one FP32 kick of nv = 8192 by 3 dk dt:
+// 7.8e-7 off in f, with the new start 4.0e-7, with 8 bins per thread 5.9e-7).
 template <class T>
 struct PhaseMul {
   T C, S;
-  cx<T> cur, step;
+  cx<T> cur, step, mid;  // mid: cur of the 9th of 16 bins
   VP_HD PhaseMul() {}
   VP_HD PhaseMul(double phi, int M, int t, int TPT) {
     cx<T> h;
@@ -498,6 +507,10 @@ struct PhaseMul {
     cis_neg((double)t * phi, cur);
     cur = mul(cur, half_phase(C, S, T(1) / T(M)));
     cis_neg((double)TPT * phi, step);
+    if (M / TPT == 16) {
+      cis_neg((double)(t + 8 * TPT) * phi, mid);
+      mid = mul(mid, half_phase(C, S, T(1) / T(M)));
+    }
   }
 };
 
@@ -537,6 +550,7 @@ template <class T>
 struct BgPhaseMul {
   T C, S;
   cx<T> cm, cs, qm;  // P_t - 1, P_TPT - 1, exp(i (TPT - t) phi) - 1
+  cx<T> cm8, qm7;    // of 16 bins: P_k - 1 of the 9th, exp(i (M - k) phi) - 1 of the 8th
   const cx<T>* bhat;
   VP_HD BgPhaseMul() {}
   VP_HD BgPhaseMul(double phi, int M, int t, int TPT, const cx<T>* bhat_) : bhat(bhat_) {
@@ -547,6 +561,10 @@ struct BgPhaseMul {
     cm = cis_neg_m1<T>((double)t * phi);
     cs = cis_neg_m1<T>((double)TPT * phi);
     qm = cis_neg_m1<T>((double)(t - TPT) * phi);
+    if (M / TPT == 16) {
+      cm8 = cis_neg_m1<T>((double)(t + 8 * TPT) * phi);
+      qm7 = cis_neg_m1<T>((double)(t - 9 * TPT) * phi);
+    }
   }
 };
 
@@ -622,7 +640,7 @@ VP_HD void couple(cx<T>* v, const cx<T>* pz, const cx<T>* wk, int t, PhaseMul<T>
     const cx<T> a = v[i];
     v[i] = mul(cur, couple_bin(m.C, m.S, wk[i], a, pz[i]));
     if (i == 0 && t == 0) v[0] = couple_dc(a, T(-2) * m.S * m.S, T(1) / T(2 * M));
-    if (i + 1 < Q) cur = mul(cur, m.step);
+    if (i + 1 < Q) cur = Q == 16 && i == 7 ? m.mid : mul(cur, m.step);
   }
 }
 
@@ -638,7 +656,7 @@ VP_HD void couple(cx<T>* v, const cx<T>* pz, const cx<T>* wk, int t, BgPhaseMul<
   cx<T> q[Q];
   q[Q - 1] = m.qm;
 #pragma unroll
-  for (int i = Q - 2; i >= 0; --i) q[i] = m1_mul(q[i + 1], csc);
+  for (int i = Q - 2; i >= 0; --i) q[i] = Q == 16 && i == 7 ? m.qm7 : m1_mul(q[i + 1], csc);
   cx<T> cm = m.cm;
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
@@ -651,7 +669,7 @@ VP_HD void couple(cx<T>* v, const cx<T>* pz, const cx<T>* wk, int t, BgPhaseMul<
       const T nyq = T(-2) * m.S * m.S;
       v[0] = add(couple_dc(a, nyq, T(1) / T(2 * M)), mk<T>(B2.re * nyq, B2.im * nyq));
     }
-    if (i + 1 < Q) cm = m1_mul(cm, m.cs);
+    if (i + 1 < Q) cm = Q == 16 && i == 7 ? m.cm8 : m1_mul(cm, m.cs);
   }
 }
 

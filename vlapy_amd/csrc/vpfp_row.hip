@@ -32,19 +32,41 @@ int launch_row_q(const vp::RowArgs<T>& a, hipStream_t s) {
   return launched();
 }
 
-// Q = 8 values per thread fills the GPU when there are many rows; with few
-// rows (fewer than ~16k threads at Q = 8) Q = 4 spreads each row over twice
-// as many threads and shortens the per-row latency chain.
+// Values per thread for `rows` rows of M points.  8 fill the GPU when there are
+// many rows; with few (fewer than ~16k threads at 8) 4 spread each row over
+// twice as many threads and shorten the per-row latency chain.  16 where 8 leave
+// too few workgroups on a CU for one to exchange through LDS while another
+// computes (times of four steps, 8 against 16 values):
+//   FP32 M = 4096: one workgroup of 512 threads fits a CU, or two of 256.  With
+//     more rows than CUs 16: 1024 rows 470 -> 362 us, 512 rows 285 -> 235 (256
+//     rows 166 either way); delta-f 1024 rows 562 -> 433.  E stays as accurate
+//     (relative error after four steps 4.2e-7 both, without collisions 6.2e-7 and
+//     3.5e-7), f too (7.0e-7 and 6.9e-7; with collisions 6.6e-7 and 8.0e-7).
+//   FP32 M = 2048: 8.  16 take 250 -> 229 us at 1024 rows, 409 -> 401 at 2048, but
+//     lose at 512 (154, 163) and with delta-f (2048 rows 475, 545).
+//   FP64: 8 (M = 4096 at 16 values spills 260 bytes at two workgroups per CU:
+//     1024 rows 649 and 652; M = 2048 310 and 314).
+template <class T, int M, bool BG>
+constexpr bool has_q16 = M <= 4096 && (BG ? sizeof(T) == 4 && M == 4096 : M >= 256);
+
+template <class T, int M, bool BG>
+int row_rule(long long rows) {
+  if (M == 4096 && sizeof(T) == 4 && rows > 256) return 16;
+  if (M >= 16 && M <= 2048 && rows * (M / 8) < 16384) return 4;
+  return 8;
+}
+
 // q: 4, 8 or 16 forces that many values per thread (where it exists: 4 for
 // 16 <= M <= 2048, 16 for M >= 256; delta-f rows: 4 or 8, q = 16 runs at
-// 8), 0 = the row-count rule above
+// 8 in FP64 and below M = 4096), 0 = row_rule
 template <class T, int M, bool BG>
 int launch_row(const vp::RowArgs<T>& a, hipStream_t s, int q) {
-  if constexpr (!BG && M >= 256 && M <= 4096) {
+  if (q == 0) q = row_rule<T, M, BG>(a.nx);
+  if constexpr (has_q16<T, M, BG>) {
     if (q == 16) return launch_row_q<T, M, 16, BG>(a, s);
   }
   if constexpr (M >= 16 && M <= 2048) {
-    if (q == 4 || (q == 0 && (long long)a.nx * (M / 8) < 16384)) return launch_row_q<T, M, 4, BG>(a, s);
+    if (q == 4) return launch_row_q<T, M, 4, BG>(a, s);
   }
   return launch_row_q<T, M, qfor(M), BG>(a, s);
 }
@@ -89,11 +111,12 @@ template <class T, int M, bool BG>
 int launch_row_multi(const vp::RowMulti<T>& m, hipStream_t s, int q) {
   long long rows = 0;
   for (int i = 0; i < m.nseg; ++i) rows += m.seg[i].rows;
-  if constexpr (!BG && M >= 256 && M <= 4096) {
+  if (q == 0) q = row_rule<T, M, BG>(rows);
+  if constexpr (has_q16<T, M, BG>) {
     if (q == 16) return launch_row_multi_q<T, M, 16, BG>(m, s);
   }
   if constexpr (M >= 16 && M <= 2048) {
-    if (q == 4 || (q == 0 && rows * (M / 8) < 16384)) return launch_row_multi_q<T, M, 4, BG>(m, s);
+    if (q == 4) return launch_row_multi_q<T, M, 4, BG>(m, s);
   }
   return launch_row_multi_q<T, M, qfor(M), BG>(m, s);
 }
