@@ -510,6 +510,7 @@ __global__ __launch_bounds__(kBT) void k_bwd_out(const float* dy, const bf16* a3
     if (t < kNV) nd = dy[(size_t)row * kNV + t];
   };
   fetch(blockIdx.x);
+  __syncthreads();  // R cleared before any thread writes a record
   for (int row = blockIdx.x; row < rows; row += gridDim.x) {
     bf16x8 v3[4];
 #pragma unroll
