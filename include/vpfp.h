@@ -92,7 +92,8 @@ int vpfp_edfdv(vpfp_plan_t plan, const void* f_in, void* f_out, const double* e,
 int vpfp_compute_charges(vpfp_plan_t plan, const void* f, double* n_out, void* stream);
 
 /* E = Re ifft(i one_over_kx fft(1 - n)).  Replaces field.solve_for_field,
- * field.py:52-63.  Any nx >= 2 (direct DFT when nx is not a power of two). */
+ * field.py:52-63.  Any nx in [2, 4096] (direct DFT when nx is not a power of
+ * two).  e_out may be charge_density. */
 int vpfp_solve_for_field(vpfp_plan_t plan, const double* charge_density, double* e_out, void* stream);
 
 /* E = driver + solve_for_field(compute_charges(f)).  Replaces
@@ -111,8 +112,8 @@ int vpfp_field(vpfp_plan_t plan, const void* f, const double* driver, double* e_
  * ends and shared by every call on that GPU: calls that overlap on one GPU
  * race.  nx > VPFP_NOALLOC_MAX_NX is refused with VPFP_EBADARG.  Power-of-two
  * nx >= 4 takes the FFT field kernel (one workgroup), any other nx the direct
- * DFT, as vpfp_field does; the twiddles are formed on the device (sincospi),
- * so results agree with vpfp_field to rounding, not bit for bit. */
+ * DFT, as vpfp_solve_for_field does; the twiddles are formed on the device
+ * (sincospi), so results agree with vpfp_field to rounding, not bit for bit. */
 #define VPFP_NOALLOC_MAX_NX 4096
 #define VPFP_NOALLOC_SCRATCH_BYTES 98304
 int vpfp_field_noalloc(int nx, int nv, int precision, double dv, const double* one_over_kx, const void* f,

@@ -767,7 +767,7 @@ int do_density(vpfp_plan_t p, const void* f, double scale, double* part, hipStre
   return launch_density<T>(f, p->nx, p->nv, scale, part, s);
 }
 
-// the plan's field solves outside a step: any nx <= 4096
+// vpfp_field's solve: any nx <= 4096
 int green_dispatch(const vp::FieldArgs& a, hipStream_t s) {
   if (!a.green) return fail(VPFP_EUNSUPPORTED, "nx must be at most 4096 for the field solve");
   hipLaunchKernelGGL(k_green, dim3((a.nx + 3) / 4), dim3(256), 0, s, a);
@@ -1934,7 +1934,13 @@ int vpfp_solve_for_field(vpfp_plan_t p, const double* n, double* e_out, void* st
   if (int rc = check_plan(p)) return rc;
   if (!n || !e_out) return fail(VPFP_EBADARG, "null array");
   if (p->nx < 2) return fail(VPFP_EUNSUPPORTED, "nx must be at least 2");
-  return green_dispatch(field_args(p, n, 1, 1.0, nullptr, e_out, nullptr, nullptr, false), p->streams.use(stream));
+  // transformed, not summed with the Green's function: the density is staged
+  // before any E is written (e_out may be n), and a given n keeps the accuracy of
+  // its bins (period 4, nx = 4096: E exact; the sum, evaluated in 64 bits, is
+  // 5e-14 of it off).  The sum is for densities formed here, whose own rounding
+  // is as large.
+  const bool pow2 = p->nx_pow2 && p->nx >= 4 && p->nx <= 4096;
+  return field_dispatch(field_args(p, n, 1, 1.0, nullptr, e_out, nullptr, nullptr, pow2), pow2, p->streams.use(stream));
 }
 
 int vpfp_field(vpfp_plan_t p, const void* f, const double* driver, double* e_out, void* stream) {

@@ -283,8 +283,8 @@ VP_HD void series_body(Ctx& c, const double* e, const double* driver, int nx, do
   }
 }
 
-// E(x) = driver(x) + sum_j g_{x-j} rho_j at any nx, one wavefront per x (the
-// plan's own field solves): nx = 100 2.7 us where the direct transform on one
+// E(x) = driver(x) + sum_j g_{x-j} rho_j at any nx, one wavefront per x
+// (vpfp_field): nx = 100 2.7 us where the direct transform on one
 // workgroup took 22.5
 template <class Ctx>
 VP_HD void green_body(Ctx& c, const FieldArgs& a) {
