@@ -142,7 +142,8 @@ int vpfp_collide(vpfp_plan_t plan, const void* f_in, void* f_out, void* stream);
  * driver [n_steps][nx] (field added at step i) may be NULL.
  * e_hist [n_steps][nx], moments [n_steps][VPFP_NMOMENTS][nx] (trapz moments
  * of f after the step) and series [n_steps][2] (mean E^2, mean driver^2) are
- * optional outputs (NULL to skip). */
+ * optional outputs (NULL to skip).  e_hist may be driver, a step's E replacing
+ * its driver (one more launch per step). */
 int vpfp_step_n(vpfp_plan_t plan, void* f, double* e, int n_steps, const double* driver, double* e_hist,
                 double* moments, double* series, void* stream);
 

@@ -809,6 +809,21 @@ struct StepTail {
   }
 };
 
+// n doubles at a and m at b (either may be null) share memory
+bool overlap(const double* a, size_t n, const double* b, size_t m) {
+  const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return a && b && x < y + m * sizeof(double) && y < x + n * sizeof(double);
+}
+
+// The drivers lie where the fields are written (e_hist in their place, or e).
+// The row kernel then cannot form the field: its waves read a driver that one
+// of them overwrites, and the series are taken from drivers a launch after E has
+// replaced them.  A field launch of its own reads each before it writes.
+bool drivers_overwritten(vpfp_plan_t p, const double* driver, size_t n_drv, const double* e_hist, size_t n,
+                         const double* e) {
+  return overlap(driver, n_drv * p->nx, e_hist, n * p->nx) || overlap(driver, n_drv * p->nx, e, p->nx);
+}
+
 // the last step's tail and e <- E
 template <class T>
 int finish_steps(vpfp_plan_t p, const StepTail<T>& tail, int n_modes, const double* e_cur, double* e, hipStream_t s) {
@@ -865,7 +880,8 @@ int do_step_n(vpfp_plan_t p, void* f, double* e, int n, const double* driver, do
   if (n <= 0) return prof_collect(p->prof);
   const bool coll = p->nu > 0.0;
   const double half = 0.5 * p->dt;
-  const int mode = field_mode(p);
+  int mode = field_mode(p);
+  if (mode >= kFieldRows && drivers_overwritten(p, driver, n, e_hist, n, e)) mode = kFieldLaunch;
   if (p->fuse == 2 && p->nx > kFuseRowsNx)
     return fail(VPFP_EUNSUPPORTED, "field in the row kernel needs nx <= " + std::to_string(kFuseRowsNx));
   auto ra = row_args<T>(p, f, f);
@@ -967,6 +983,7 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
   // every field solve is formed by the row launch that follows it, by the size
   // rule (the tuning's other forms are for the leapfrog step)
   const bool sum = rule_mode(p) == kFieldRowsSum;
+  const bool own = drivers_overwritten(p, driver, (size_t)n * kSchemeFields, e_hist, n, e);  // field launches
   const double* e_cur = e;
   long long field_no = 0;
   StepTail<T> tail;
@@ -997,7 +1014,10 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
       const bool last = j == kSchemeFields - 1;
       double* eo = (last && e_hist) ? e_hist + (size_t)i * p->nx : p->ering + (size_t)(field_no & 1) * p->nx;
       drv = driver ? driver + ((size_t)i * kSchemeFields + j) * p->nx : nullptr;
-      if (sum)
+      if (own) {
+        double* ser = last && series ? series + 2 * (size_t)i : nullptr;
+        PROF(KK_FIELD, field_dispatch(field_args(p, p->dens, p->ntiles, p->dv, drv, eo, nullptr, ser, true), true, s));
+      } else if (sum)
         PROF(KK_FIELD, rows_field(p, &next, drv, eo, true, s));
       else if (int rc = rows_field(p, &next, drv, eo, false, s))
         return rc;
@@ -1017,13 +1037,13 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
                               : reinterpret_cast<T*>(f_store) + (size_t)i * p->nx * p->nv;
     if (rb.flags || rb.f_copy) {
       PROF(KK_ROW, row_dispatch<T>(rb, s, p->row_q));
-    } else {
+    } else if (!own) {
       // PEFRL without a collision or outputs ends with its field: no row launch
       PROF(KK_FIELD, field_dispatch(field_args(p, p->dens, p->ntiles, p->dv, drv, rb.fld.e_out, nullptr, nullptr, true), true, s));
     }
     tail.e = e_cur;
     tail.drv = drv;
-    tail.series = series ? series + 2 * (size_t)i : nullptr;
+    tail.series = series && !own ? series + 2 * (size_t)i : nullptr;
     if (f_store && n_modes > 0) {
       tail.xm_f = rb.f_copy;
       tail.xm_out = reinterpret_cast<cx<double>*>(f_store) + (size_t)i * n_modes * p->nv;
