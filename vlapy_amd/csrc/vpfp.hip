@@ -980,10 +980,11 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
   const int ns = (int)st.size();
   const bool coll = p->nu > 0.0;
   const bool first_kick = st[0].kick, last_kick = st[ns - 1].kick;
-  // every field solve is formed by the row launch that follows it, by the size
-  // rule (the tuning's other forms are for the leapfrog step)
+  // every field is formed by the row launch that follows it, by the size rule
+  // (the tuning's other forms are for the leapfrog step); a field that no row
+  // launch follows, or that replaces a driver, by a launch of its own
   const bool sum = rule_mode(p) == kFieldRowsSum;
-  const bool own = drivers_overwritten(p, driver, (size_t)n * kSchemeFields, e_hist, n, e);  // field launches
+  const bool shared = drivers_overwritten(p, driver, (size_t)n * kSchemeFields, e_hist, n, e);
   const double* e_cur = e;
   long long field_no = 0;
   StepTail<T> tail;
@@ -998,6 +999,12 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
     int j = 0;  // field solve of this step
     vp::RowArgs<T> next = row_args<T>(p, f, f);  // the next row launch, with the field it forms
     const double* drv = nullptr;
+    bool own = false;  // the last field solve had a launch of its own
+    // the row launch that ends the step, and whether it has anything to do: PEFRL
+    // without a collision or outputs ends with its field
+    const int end_flags = (last_kick ? vp::RK_KICK_A : 0) | (coll ? vp::RK_COLLIDE : 0) |
+                          (moments ? vp::RK_MOMENTS : 0) | (first_kick && i + 1 < n ? vp::RK_KICK_B : 0);
+    const bool end_row = end_flags || f_store;
     for (int k = 0; k < ns; ++k) {
       const Stage& g = st[k];
       if (g.kick) {
@@ -1014,6 +1021,7 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
       const bool last = j == kSchemeFields - 1;
       double* eo = (last && e_hist) ? e_hist + (size_t)i * p->nx : p->ering + (size_t)(field_no & 1) * p->nx;
       drv = driver ? driver + ((size_t)i * kSchemeFields + j) * p->nx : nullptr;
+      own = shared || (last && !end_row);
       if (own) {
         double* ser = last && series ? series + 2 * (size_t)i : nullptr;
         PROF(KK_FIELD, field_dispatch(field_args(p, p->dens, p->ntiles, p->dv, drv, eo, nullptr, ser, true), true, s));
@@ -1030,17 +1038,11 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
     rb.dt_a = last_kick ? st[ns - 1].c * p->dt : 0.0;
     rb.dt_b = st[0].c * p->dt;
     rb.moments = moments ? moments + (size_t)i * vp::kMoments * p->nx : nullptr;
-    rb.flags = (last_kick ? vp::RK_KICK_A : 0) | (coll ? vp::RK_COLLIDE : 0) | (moments ? vp::RK_MOMENTS : 0) |
-               (first_kick && i + 1 < n ? vp::RK_KICK_B : 0);
+    rb.flags = end_flags;
     if (f_store)
       rb.f_copy = n_modes > 0 ? reinterpret_cast<T*>(p->fcopy) + (size_t)(i & 1) * p->nx * p->nv
                               : reinterpret_cast<T*>(f_store) + (size_t)i * p->nx * p->nv;
-    if (rb.flags || rb.f_copy) {
-      PROF(KK_ROW, row_dispatch<T>(rb, s, p->row_q));
-    } else if (!own) {
-      // PEFRL without a collision or outputs ends with its field: no row launch
-      PROF(KK_FIELD, field_dispatch(field_args(p, p->dens, p->ntiles, p->dv, drv, rb.fld.e_out, nullptr, nullptr, true), true, s));
-    }
+    if (end_row) PROF(KK_ROW, row_dispatch<T>(rb, s, p->row_q));
     tail.e = e_cur;
     tail.drv = drv;
     tail.series = series && !own ? series + 2 * (size_t)i : nullptr;
