@@ -601,9 +601,10 @@ int scan_tiles_per_wg(long long tiles) { return tiles >= 4 * 2048 ? 4 : tiles >=
 // than its LDS holds, they are summed once first.
 enum FieldMode { kFieldLaunch = 0, kFieldTail = 1, kFieldRows = 2, kFieldRowsSum = 3 };
 constexpr int kFuseRowsNx = 128;  // fuse_field 2
-int rule_mode(vpfp_plan_t p) {
-  return p->nx <= vp::kProNx && (long long)p->ntiles * p->nx <= vp::kProSum ? kFieldRows : kFieldRowsSum;
+int rule_mode(int nx, int ntiles) {
+  return nx <= vp::kProNx && (long long)ntiles * nx <= vp::kProSum ? kFieldRows : kFieldRowsSum;
 }
+int rule_mode(vpfp_plan_t p) { return rule_mode(p->nx, p->ntiles); }
 int field_mode(vpfp_plan_t p) { return p->fuse >= 0 ? p->fuse : rule_mode(p); }
 
 enum KernelKind { KK_ROW = 0, KK_DRIFT = 1, KK_FIELD = 2, KK_OTHER = 3 };
@@ -1211,9 +1212,10 @@ int batch_step_n(vpfp_batch_s* b, void* f, double* e, int n, double* series, hip
 
 // ---------------------------------------------------------------- autotuner
 // Times every valid launch shape of the step on scratch state and keeps the
-// fastest: values per thread of the row kernels (4 or 8, where both exist),
-// columns per drift workgroup (4, 8, 16) and, for a single grid with
-// nx <= 256, the field solve as a drift tail or as its own launch.
+// fastest: values per thread of the row kernels (row_q_candidates), columns per
+// drift tile (4, 8, 16, 32), tiles per drift workgroup (1, 2, 4) and their order,
+// the MFMA drift and, for a single grid, where the field is solved (FieldMode;
+// -1, the size rule, where that is neither of the others).
 
 // (1 + 0.01 cos(2 pi x / nx)) exp(-v^2 / 2) / sqrt(2 pi) on every row
 template <class T>
@@ -1340,12 +1342,14 @@ int autotune_plan(vpfp_plan_t p, int n_steps, hipStream_t s) {
       if (C > p->nv) continue;
       for (int fuse : {0, 1, 2, -1}) {
         if (fuse == 1 && p->nx > 256) continue;
-        if (fuse == -1 && p->nx <= kFuseRowsNx) continue;  // fuse 2 is the rule's choice there
         if (fuse == 2 && p->nx > kFuseRowsNx) continue;
         for (int xo : {0, 1})
           for (int dt : {1, 2, 4}) {
             // more tiles per workgroup only where it changes the grid
             if (dt > 1 && p->nv / C / dt < 8) continue;
+            // the rule's choice is tried as 2 where it is that
+            if (fuse == -1 && p->nx <= kFuseRowsNx && rule_mode(p->nx, drift_wgs(p->nv, C, dt, false)) == kFieldRows)
+              continue;
             cands.push_back({q, C, fuse, xo, dt, 0});
             // the MFMA drift (no drift tail)
             if (p->dft_mat && (C == 16 || C == 32) && fuse != 1) cands.push_back({q, C, fuse, xo, dt, 1});
