@@ -878,13 +878,13 @@ int do_tri(vpfp_plan_t p, const double* A, const double* B, const double* Cc, co
 template <class T>
 int do_step_n(vpfp_plan_t p, void* f, double* e, int n, const double* driver, double* e_hist, double* moments,
               double* series, hipStream_t s, void* f_store = nullptr, int n_modes = 0) {
-  if (n <= 0) return prof_collect(p->prof);
   const bool coll = p->nu > 0.0;
   const double half = 0.5 * p->dt;
   int mode = field_mode(p);
   if (mode >= kFieldRows && drivers_overwritten(p, driver, n, e_hist, n, e)) mode = kFieldLaunch;
   if (p->fuse == 2 && p->nx > kFuseRowsNx)
     return fail(VPFP_EUNSUPPORTED, "field in the row kernel needs nx <= " + std::to_string(kFuseRowsNx));
+  if (n <= 0) return prof_collect(p->prof);
   auto ra = row_args<T>(p, f, f);
   ra.e = e;
   ra.dt_a = half;
