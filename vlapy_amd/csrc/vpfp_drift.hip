@@ -118,7 +118,7 @@ __global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg)) void k_drift(vp::Dr
   vp::drift_body<T, M, Q, C, false, unsigned long>(c, lds, a);  // any nv
 }
 
-// one column tile per workgroup (nv at most kDriftMaxWG tiles of 32)
+// one column tile per workgroup, offsets of 32 bits (offsets32)
 template <class T, int M, int Q, int C>
 __global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg), (vp::DriftCfg<T, M, Q, C>::min_waves)) void k_drift_one(
     vp::DriftArgs<T> a) {
@@ -127,11 +127,19 @@ __global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg), (vp::DriftCfg<T, M,
   vp::drift_body<T, M, Q, C, true, unsigned>(c, lds, a);
 }
 
+// the largest offset of a lane from its tile's first value, column C - 1 of row
+// 2 (TPT - 1), in bytes
+template <class T, class Cfg, int C>
+constexpr bool offsets32(long long nv) {
+  return (2LL * (Cfg::wg / C - 1) * nv + C) * (long long)sizeof(T) <= 0xffffffffLL;
+}
+
 template <class T, int M, int C>
 int launch_drift_c(const vp::DriftArgs<T>& a, hipStream_t s, int gx, int gy) {
   constexpr int Q = vp::drift_q<T>(M);
   using Cfg = vp::DriftCfg<T, M, Q, C>;
-  auto kern = a.nv == gx * C ? k_drift_one<T, M, Q, C> : k_drift<T, M, Q, C>;
+  const bool one = a.nv == (long long)gx * C && offsets32<T, Cfg, C>(a.nv);
+  auto kern = one ? k_drift_one<T, M, Q, C> : k_drift<T, M, Q, C>;
   if (Cfg::wg > 1024 || Cfg::lds > kMaxLds)
     return fail(VPFP_EUNSUPPORTED, "drift tile of " + std::to_string(C) + " columns does not fit a workgroup");
   if (a.fuse_field && !Cfg::tail) return fail(VPFP_EUNSUPPORTED, "field tail not available at this size");
@@ -175,6 +183,7 @@ __global__ __launch_bounds__((vp::DriftCfg<T, M, Q, C>::wg)) void k_drift_multi(
   // nv <= 8192.  64-bit offsets for the longer columns all the same (nx = 128
   // FP32, 4096 instances: 280 us, with 32-bit ones 288; nx = 64: 124 and 114)
   using Off = std::conditional_t<(M <= 32), unsigned, unsigned long>;
+  static_assert(M > 32 || offsets32<T, vp::DriftCfg<T, M, Q, C>, C>(8192), "32-bit offsets");
   vp::drift_body<T, M, Q, C, false, Off>(c, lds, a);
 }
 
