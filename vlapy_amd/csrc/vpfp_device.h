@@ -263,17 +263,13 @@ VP_HD constexpr double cos32(int J) {
 }
 VP_HD constexpr double sin32(int J) { return cos32(J - 8); }
 
-// b * W_32^J  (forward: W = exp(-2 pi i J / 32); inverse: conjugate)
+// b * W_32^J for J = 0, 8, 16 or 24 (forward: W = exp(-2 pi i J / 32); inverse: conjugate)
 template <bool INV, class T>
-VP_HD cx<T> tw32(cx<T> b, int J) {
-  J &= 31;
+VP_HD cx<T> quarter_turns(cx<T> b, int J) {
   if (J == 0) return b;
   if (J == 16) return mk<T>(-b.re, -b.im);
   if (J == 8) return INV ? mk<T>(-b.im, b.re) : mk<T>(b.im, -b.re);
-  if (J == 24) return INV ? mk<T>(b.im, -b.re) : mk<T>(-b.im, b.re);
-  const T c = (T)cos32(J), s = (T)sin32(J);
-  return INV ? mk<T>(b.re * c - b.im * s, b.im * c + b.re * s)
-             : mk<T>(b.re * c + b.im * s, b.im * c - b.re * s);
+  return INV ? mk<T>(b.im, -b.re) : mk<T>(-b.im, b.re);
 }
 
 template <int R>
@@ -286,41 +282,49 @@ VP_HD constexpr int brev(int i) {
   return r;
 }
 
-// (a, b) <- (a + W b, a - W b) with W = W_32^J (inverse: its conjugate).  For
-// a W off the axes one of its parts is factored out, W b = c (b' + i b'') with
-// c the larger part, so that c goes into the two sums as their fma: 6
-// instructions instead of the 8 of a product and two sums.
+VP_HD float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
+VP_HD double fma_t(double a, double b, double c) { return fma(a, b, c); }
+
+// (a, b) <- (a + W b, a - W b) with W = W_32^J (inverse: its conjugate), in 6
+// instructions at odd multiples of 45 degrees, whose factor goes into the two
+// sums as their fma, instead of the 8 of a product and two sums.
+//
+// The other angles (radix 16) take 10, with the larger part of W as 1 - g: a
+// rounded cos(pi/8) is the same 3e-8 off in every transform, so its error grows
+// with the steps as nothing random does, and 1 - g with a rounded g is 2e-9 off.
+// Rows of nv = 8192 in FP32 at 16 values, collisions, f after 4 and 12 steps:
+// 8.05e-7 and 2.18e-6 off with tan(pi/8) and the rounded larger part factored out
+// (6 instructions, four steps of 1024 rows 364 us), 5.9e-7 and 1.50e-6 so
+// (366 to 368 us); 8 values, which have multiples of 45 degrees only, 6.6e-7 and 1.67e-6.
 template <bool INV, class T>
 VP_HD void butterfly(cx<T>& a, cx<T>& b, int J) {
   J &= 31;
+  const cx<T> x = a;
   if ((J & 7) == 0) {
-    const cx<T> w = tw32<INV>(b, J), x = a;
+    const cx<T> w = quarter_turns<INV>(b, J);
     a = add(x, w);
     b = sub(x, w);
     return;
   }
+  // W b = (b.re cd + b.im sd, b.im cd - b.re sd)
   const double cd = cos32(J), sd = INV ? -sin32(J) : sin32(J);
-  const bool cbig = (cd < 0 ? -cd : cd) >= (sd < 0 ? -sd : sd);
-  // r from the rounded f so that f^2 (1 + r^2) = 1 as near as r allows: the two
-  // transforms of a pusher multiply by W and its conjugate, so an error of the
-  // angle drops out and one of the modulus scales modes, step after step (FP32
-  // rows at 16 values, whose W are not only multiples of 45 degrees)
-  const double big = cbig ? cd : sd, small = cbig ? sd : cd;
-  const T f = (T)big;
-  const T r = (T)((small + (big - (double)f) * (big + (double)f) / (2.0 * small)) / (double)f);
-  // W b = (b.re c + b.im s, b.im c - b.re s)
-  const bool one = (J & 3) == 0 && r > T(0), mone = (J & 3) == 0 && r < T(0);  // odd multiples of 45 degrees
-  T u, w;
-  if (cbig) {
-    u = one ? b.re + b.im : mone ? b.re - b.im : b.re + r * b.im;
-    w = one ? b.im - b.re : mone ? b.im + b.re : b.im - r * b.re;
-  } else {
-    u = b.im + r * b.re;
-    w = r * b.im - b.re;
+  if ((J & 3) == 0) {
+    const T f = (T)cd;
+    const bool same = (cd > 0) == (sd > 0);
+    const T u = same ? b.re + b.im : b.re - b.im, w = same ? b.im - b.re : b.im + b.re;
+    a = mk<T>(x.re + f * u, x.im + f * w);
+    b = mk<T>(x.re - f * u, x.im - f * w);
+    return;
   }
-  const cx<T> x = a;
-  a = mk<T>(x.re + f * u, x.im + f * w);
-  b = mk<T>(x.re - f * u, x.im - f * w);
+  // W b = sg (p - g p + h q), p the turn of b by the axis next to W, q by the other
+  const bool cbig = cd * cd > sd * sd;
+  const double big = cbig ? cd : sd, small = cbig ? sd : cd;
+  const bool pos = big > 0;
+  const T g = (T)(1.0 - (pos ? big : -big)), h = (T)(pos ? small : -small);
+  const cx<T> r = mk<T>(b.im, -b.re), p = cbig ? b : r, q = cbig ? r : b;
+  const T u = p.re + fma_t(h, q.re, -g * p.re), w = p.im + fma_t(h, q.im, -g * p.im);
+  a = pos ? mk<T>(x.re + u, x.im + w) : mk<T>(x.re - u, x.im - w);
+  b = pos ? mk<T>(x.re - u, x.im - w) : mk<T>(x.re + u, x.im + w);
 }
 
 template <int R, bool INV, class T>
@@ -466,8 +470,6 @@ VP_HD void fft(Ctx& c, cx<T>* v, cx<T>* buf, const Tw<T>& tw, int t, bool act = 
 // expression below times (C - i S) (C + i S) / M: dividing by the rounded
 // norm keeps the pushers from scaling every mode by the same rounding error
 // step after step, and what is left of the error of C and S is one of P_M.
-VP_HD float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
-VP_HD double fma_t(double a, double b, double c) { return fma(a, b, c); }
 template <class T>
 VP_HD cx<T> half_phase(T C, T S, T s) {
   const T e = C * C > T(0.5) ? fma_t(S, S, fma_t(C, C, T(-1))) : fma_t(C, C, fma_t(S, S, T(-1)));

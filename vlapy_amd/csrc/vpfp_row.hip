@@ -38,10 +38,11 @@ int launch_row_q(const vp::RowArgs<T>& a, hipStream_t s) {
 // too few workgroups on a CU for one to exchange through LDS while another
 // computes (times of four steps, 8 against 16 values):
 //   FP32 M = 4096: one workgroup of 512 threads fits a CU, or two of 256.  With
-//     more rows than CUs 16: 1024 rows 470 -> 362 us, 512 rows 285 -> 235 (256
-//     rows 166 either way); delta-f 1024 rows 562 -> 433.  E stays as accurate
-//     (relative error after four steps 4.2e-7 both, without collisions 6.2e-7 and
-//     3.5e-7), f too (7.0e-7 and 6.9e-7; with collisions 6.6e-7 and 8.0e-7).
+//     more rows than CUs 16: 1024 rows 469 -> 366 us, 512 rows 284 -> 239 (256
+//     rows 165 and 168); delta-f 561 -> 438 and 328 -> 272.  No less accurate: f
+//     after four steps with collisions 6.6e-7 and 5.9e-7 off, without 7.1e-7 and
+//     5.8e-7, delta-f 7.6e-7 and 7.1e-7; E 4.7e-7 and 4.6e-7, 4.6e-7 and 4.0e-7,
+//     1.7e-7 and 1.6e-7 (means over 8 initial states).
 //   FP32 M = 2048: 8.  16 take 250 -> 229 us at 1024 rows, 409 -> 401 at 2048, but
 //     lose at 512 (154, 163) and with delta-f (2048 rows 475, 545).
 //   FP64: 8 (M = 4096 at 16 values spills 260 bytes at two workgroups per CU:
