@@ -155,9 +155,10 @@ int vpfp_step_n(vpfp_plan_t plan, void* f, double* e, int n_steps, const double*
  *                 next half kick, no extra launch);
  *   n_modes > 0:  the first n_modes Fourier modes along x of f, f_store
  *                 [n_steps][n_modes][nv] complex128, equal to vpfp_x_modes:
- *                 the row kernel writes f to plan scratch and extra
- *                 workgroups of the next step's row launch sum it over x
- *                 (one more launch after the last step).
+ *                 the row kernel writes f to plan scratch (two copies of f,
+ *                 nx nv values each, allocated at the plan's first such call)
+ *                 and extra workgroups of the next step's row launch sum it
+ *                 over x (one more launch after the last step).
  * Two launches per step either way (three where the field's densities are
  * summed first).  Under delta-f storage the store holds
  * f itself. */

@@ -6,12 +6,15 @@
 // vpfp_drift.hip (one object per storage type, compiled in parallel).
 //
 // Launch shapes (wave64):
-//   row kernel   M = nv/2 complex points per row, Q = min(8, M) per thread,
-//                TPT = M/Q threads per row, max(1, 64/TPT) rows per workgroup
-//   drift kernel M = nx/2, Q = min(8, M), TPT = M/Q threads per column,
-//                C columns per workgroup (16 for nx <= 256, 8 for nx = 512,
-//                4 above), one partial density row per workgroup
-//   field kernel one workgroup of 256 threads
+//   row kernel   M = nv/2 complex points per row, Q = 4, 8 or 16 per thread
+//                (row_rule in vpfp_row.hip), TPT = M/Q threads per row,
+//                max(1, 64/TPT) rows per workgroup
+//   drift kernel M = nx/2, Q = 4 or 8 (drift_q), TPT = M/Q threads per column,
+//                tiles of C columns (drift_tile, scan_tile), one or more tiles
+//                and one partial density row per workgroup
+//   field kernel workgroups of 256 threads, one per grid or instance (nx/64 for
+//                single grids of nx >= 128); the fused step of a single grid
+//                forms its field in the row kernel (FieldMode)
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -698,7 +701,7 @@ vp::DriftArgs<T> drift_args(vpfp_plan_t p, const void* fin, void* fout, double d
 }
 
 vp::FieldArgs field_args(vpfp_plan_t p, const double* part, int ntiles, double scale, const double* driver,
-                         double* e_out, double* e_out2, double* series, bool pow2) {
+                         double* e_out, double* series, bool pow2) {
   vp::FieldArgs a;
   std::memset(&a, 0, sizeof(a));
   a.part = part;
@@ -711,7 +714,6 @@ vp::FieldArgs field_args(vpfp_plan_t p, const double* part, int ntiles, double s
   a.tw = pow2 ? p->tw_xs : p->tw_xd;
   a.driver = driver;
   a.e_out = e_out;
-  a.e_out2 = e_out2;
   a.series = series;
   a.series_stride = 0;
   a.green = p->green;
@@ -786,7 +788,7 @@ int rows_field(vpfp_plan_t p, vp::RowArgs<T>* ra, const double* drv, double* e_o
     hipLaunchKernelGGL(k_rho, dim3(p->nx / XS), dim3(kFT), 0, s, p->dens, p->ntiles, p->nx, p->rho_g);
     if (int rc = launched()) return rc;
   }
-  ra->fld = field_args(p, sum ? p->rho_g : p->dens, sum ? 1 : p->ntiles, p->dv, drv, e_out, nullptr, nullptr, false);
+  ra->fld = field_args(p, sum ? p->rho_g : p->dens, sum ? 1 : p->ntiles, p->dv, drv, e_out, nullptr, false);
   return VPFP_OK;
 }
 
@@ -901,12 +903,12 @@ int do_step_n(vpfp_plan_t p, void* f, double* e, int n, const double* driver, do
     if (mode == kFieldTail) {
       auto da = drift_args<T>(p, f, f, p->dt, p->dens);
       da.fuse_field = 1;
-      da.fld = field_args(p, p->dens, p->ntiles, p->dv, drv, ei, nullptr, ser, true);
+      da.fld = field_args(p, p->dens, p->ntiles, p->dv, drv, ei, ser, true);
       PROF(KK_DRIFT, drift_dispatch<T>(da, p->C, p->ntiles, s));
     } else {
       PROF(KK_DRIFT, (do_vdfdx<T>(p, f, f, p->dt, p->dens, s)));
       if (mode == kFieldLaunch) {
-        const auto fa = field_args(p, p->dens, p->ntiles, p->dv, drv, ei, nullptr, ser, true);
+        const auto fa = field_args(p, p->dens, p->ntiles, p->dv, drv, ei, ser, true);
         PROF(KK_FIELD, field_dispatch(fa, true, s));
       } else if (mode == kFieldRowsSum) {
         PROF(KK_FIELD, rows_field(p, &rb, drv, ei, true, s));
@@ -1025,7 +1027,7 @@ int do_step_scheme(vpfp_plan_t p, int scheme, void* f, double* e, int n, const d
       own = shared || (last && !end_row);
       if (own) {
         double* ser = last && series ? series + 2 * (size_t)i : nullptr;
-        PROF(KK_FIELD, field_dispatch(field_args(p, p->dens, p->ntiles, p->dv, drv, eo, nullptr, ser, true), true, s));
+        PROF(KK_FIELD, field_dispatch(field_args(p, p->dens, p->ntiles, p->dv, drv, eo, ser, true), true, s));
       } else if (sum)
         PROF(KK_FIELD, rows_field(p, &next, drv, eo, true, s));
       else if (int rc = rows_field(p, &next, drv, eo, false, s))
@@ -1966,7 +1968,7 @@ int vpfp_solve_for_field(vpfp_plan_t p, const double* n, double* e_out, void* st
   // 5e-14 of it off).  The sum is for densities formed here, whose own rounding
   // is as large.
   const bool pow2 = p->nx_pow2 && p->nx >= 4 && p->nx <= 4096;
-  return field_dispatch(field_args(p, n, 1, 1.0, nullptr, e_out, nullptr, nullptr, pow2), pow2, p->streams.use(stream));
+  return field_dispatch(field_args(p, n, 1, 1.0, nullptr, e_out, nullptr, pow2), pow2, p->streams.use(stream));
 }
 
 int vpfp_field(vpfp_plan_t p, const void* f, const double* driver, double* e_out, void* stream) {
@@ -1975,7 +1977,7 @@ int vpfp_field(vpfp_plan_t p, const void* f, const double* driver, double* e_out
   int rc = p->prec == VPFP_F64 ? do_density<double>(p, f, p->dv, p->dens, p->streams.use(stream))
                                : do_density<float>(p, f, p->dv, p->dens, p->streams.use(stream));
   if (rc) return rc;
-  return green_dispatch(field_args(p, p->dens, 1, 1.0, driver, e_out, nullptr, nullptr, false), p->streams.use(stream));
+  return green_dispatch(field_args(p, p->dens, 1, 1.0, driver, e_out, nullptr, false), p->streams.use(stream));
 }
 
 int vpfp_field_noalloc(int nx, int nv, int precision, double dv, const double* one_over_kx, const void* f,

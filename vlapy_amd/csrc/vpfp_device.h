@@ -4,12 +4,11 @@
 // provides `tid`, `nthr` (thread index and count in the workgroup), `bid`,
 // `nblk` (workgroup index and count along x), `bidy` (workgroup index along
 // y: the instance of a batched scan), `sync()` (workgroup barrier),
-// `shfl_xor(v, mask, width)` (lane exchange inside a wavefront),
-// `add_lane<MASK>(v)` and `fold_lane<MASK>(lo, hi)` (sums of a lane pair) and,
-// for the cross-workgroup hand-off of the field kernel, `fence()` (device-scope
-// fence), `arrive(counter)` (device-scope atomic increment, returns the old
-// value), `load_coherent(p)` and `reset(counter)`.  The HIP kernels in
-// vpfp.hip instantiate it with the hardware primitives.
+// `add_lane<MASK>(v)` and `fold_lane<MASK>(lo, hi)` (sums of a lane pair),
+// `any(p)` (over a wavefront) and, for the cross-workgroup hand-off of the field
+// kernel, `fence()` (device-scope fence), `arrive(counter)` (device-scope atomic
+// increment, returns the old value) and `reset(counter)`.  GpuCtx
+// (vpfp_launch.h) provides it with the hardware primitives.
 //
 // Contents
 //   * cx<T>        : complex value in registers / LDS (T = double or float)

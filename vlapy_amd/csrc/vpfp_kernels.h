@@ -1,6 +1,6 @@
 // Kernel bodies of the VPFP step.  Each body is written for one workgroup
-// and a block context `Ctx` (tid, nthr, bid, sync, shfl_xor); vpfp.hip wraps
-// them in __global__ kernels.
+// and a block context `Ctx` (vpfp_device.h); vpfp.hip, vpfp_row.hip and
+// vpfp_drift.hip wrap them in __global__ kernels.
 //
 // Data layout (HBM): f is (nx, nv) row-major, v fastest, T = double or float.
 // A row (fixed x) is contiguous; a column (fixed v) has stride nv.
@@ -117,7 +117,6 @@ struct ArrCoef {
   }
 };
 
-// drift velocity and temperature of one row (un-normalised, trapz), chunk layout
 // trapz weight of chunk element i of thread t (rows t L .. t L + L - 1 of a
 // row of TPT L samples): 1/2 at the two ends of the row
 template <int TPT, int L>
@@ -125,6 +124,7 @@ VP_HD double chunk_w(int i, int t) {
   return ((i == 0 && t == 0) || (i == L - 1 && t == TPT - 1)) ? 0.5 : 1.0;
 }
 
+// drift velocity and temperature of one row (un-normalised, trapz), chunk layout
 template <int TPT, int L, class Ctx>
 VP_HD void coll_moments(Ctx& c, const double* d, double v0, double dvv, int N, double dv, bool dg, int t,
                         double* rs, double& vbar, double& temp) {
@@ -163,7 +163,6 @@ struct FieldArgs {
   const cx<double>* tw;   // pow2 kernel: twiddle tables of nx (Tw); DFT kernel: exp(-2 pi i n / nx), n < nx
   const double* driver;   // [nx] or null
   double* e_out;          // [nx]
-  double* e_out2;         // [nx] or null
   double* series;         // [2] or null: mean(E^2), mean(driver^2)
   int series_stride;      // batched scan: doubles between consecutive instances' series entries
   const double* green;    // [nx] Green's function of the solve (single grids; field_rows, green_body)
@@ -183,21 +182,20 @@ VP_HD FieldArgs field_instance(const FieldArgs& a, int inst) {
   r.okx += xo;
   if (r.driver) r.driver += xo;
   r.e_out += xo;
-  if (r.e_out2) r.e_out2 += xo;
   if (r.series) r.series += (size_t)inst * a.series_stride;
   return r;
 }
 
 // rho[x] = 1 - scale * sum_tiles part[tile][x] for x in [x0, x0 + XS)
 // (all FT threads; XS divides FT or FT divides XS)
-template <int FT, bool COH = false, int U = 8, class Ctx>
+template <int FT, int U = 8, class Ctx>
 VP_HD void field_density(Ctx& c, const FieldArgs& a, int x0, int XS, double* rho, double* tmp) {
   const int nx = a.nx;
   const int G = XS >= FT ? 1 : FT / XS;
   for (int l0 = c.tid; l0 < XS * G; l0 += FT) {
     const int xl = l0 % XS, g = l0 / XS;
     const double* p = a.part + x0 + xl;
-    auto ld = [&](int tl) { return COH ? c.load_coherent(p + (size_t)tl * nx) : p[(size_t)tl * nx]; };
+    auto ld = [&](int tl) { return p[(size_t)tl * nx]; };
     // U independent partial sums keep U loads in flight per thread
     double acc[U];
 #pragma unroll
@@ -254,16 +252,13 @@ VP_HD double field_rows(Ctx& c, const FieldArgs& a, unsigned char* lds, int row,
 #pragma unroll 4
     for (int j = t; j < nx; j += TPT) s[0] += a.green[(row - j) & (nx - 1)] * (1.0 - a.scale * a.part[j]);
   } else {
-    field_density<FT, false, 16>(c, a, 0, nx, rho, tmp);  // ends with a barrier
+    field_density<FT, 16>(c, a, 0, nx, rho, tmp);  // ends with a barrier
     for (int j = t; j < nx; j += TPT) s[0] += a.green[(row - j) & (nx - 1)] * rho[j];
   }
   row_sum<TPT, 1>(c, s, rs);
   if constexpr (TPT <= 64) c.sync();  // rho read before the transforms take the LDS
   const double e = s[0] + (a.driver ? a.driver[row] : 0.0);
-  if (valid && t == 0) {
-    a.e_out[row] = e;
-    if (a.e_out2) a.e_out2[row] = e;
-  }
+  if (valid && t == 0) a.e_out[row] = e;
   return e;
 }
 
@@ -623,7 +618,6 @@ VP_HD void field_finish(Ctx& c, const FieldArgs& a, int x, double ex, double* rs
   const double dr = a.driver ? a.driver[x] : 0.0;
   const double e = ex + dr;
   a.e_out[x] = e;
-  if (a.e_out2) a.e_out2[x] = e;
   acc[0] += e * e;
   acc[1] += dr * dr;
 }
@@ -639,7 +633,8 @@ struct FieldCfg {
 };
 
 // TAIL: called by the last workgroup of the drift kernel, which reads every
-// partial density row itself (coherent loads) instead of the slice hand-off
+// partial density row itself, behind its own acquire fence, instead of the slice
+// hand-off
 template <int M, int Q, int FT, bool TAIL = false, class Ctx>
 VP_HD void field_body(Ctx& c, unsigned char* lds, const FieldArgs& a) {
   using Cfg = FieldCfg<M, Q, FT>;
@@ -653,7 +648,7 @@ VP_HD void field_body(Ctx& c, unsigned char* lds, const FieldArgs& a) {
   int* flag = reinterpret_cast<int*>(lds + Cfg::lds - 16);
   if constexpr (TAIL) {
     // the caller's acquire fence makes the other workgroups' rows visible
-    field_density<FT, false>(c, a, 0, Cfg::nx, rho, tmp);
+    field_density<FT>(c, a, 0, Cfg::nx, rho, tmp);
   } else {
     if (!field_gather<FT>(c, a, rho, tmp, flag)) return;
   }

@@ -26,11 +26,6 @@ struct GpuCtx {
   __device__ __forceinline__ void fence() { __threadfence(); }
   __device__ __forceinline__ unsigned arrive(unsigned* c) { return atomicAdd(c, 1u); }
   __device__ __forceinline__ void reset(unsigned* c) { __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-  __device__ __forceinline__ double load_coherent(const double* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __device__ __forceinline__ double shfl_xor(double v, int m, int w) { return __shfl_xor(v, m, w); }
-  __device__ __forceinline__ float shfl_xor(float v, int m, int w) { return __shfl_xor(v, m, w); }
   __device__ __forceinline__ bool any(bool p) { return __any(p); }
   // v of the lane opposite in bit MASK: a DPP move for MASK < 16 (row_mirror
   // and row_half_mirror pair lane l with 15 - l and 7 - l, which also differ
