@@ -293,8 +293,9 @@ VP_HD double fma_t(double a, double b, double c) { return fma(a, b, c); }
 // with the steps as nothing random does, and 1 - g with a rounded g is 2e-9 off.
 // Rows of nv = 8192 in FP32 at 16 values, collisions, f after 4 and 12 steps:
 // 8.05e-7 and 2.18e-6 off with tan(pi/8) and the rounded larger part factored out
-// (6 instructions, four steps of 1024 rows 364 us), 5.9e-7 and 1.50e-6 so
-// (366 to 368 us); 8 values, which have multiples of 45 degrees only, 6.6e-7 and 1.67e-6.
+// (6 instructions, four steps of 1024 rows 364 us), 5.9e-7 and 1.50e-6 so (366 to
+// 368 us); 8 values, which have multiples of 45 degrees only, 6.6e-7 and 1.67e-6
+// (with the half phase in FP64 since: 5.7e-7, 1.42e-6; 6.4e-7, 1.59e-6).
 template <bool INV, class T>
 VP_HD void butterfly(cx<T>& a, cx<T>& b, int J) {
   J &= 31;

@@ -796,7 +796,7 @@ struct DriftCfg {
   // one tile per workgroup (ONE): without the next tile's values and the running
   // density in registers, two workgroups of eight waves fit a CU, and one loads
   // while the other transforms (nx = 1024, nv = 8192: FP32 36.2 -> 27.3 us; FP64,
-  // which spills 88 bytes for it, 55 -> 47)
+  // which spills 88 bytes per lane for it, 46 MB of traffic each way, 55 -> 47)
   static constexpr int min_waves = wg == 512 && 2 * lds <= 160 * 1024 ? 4 : 1;
 };
 

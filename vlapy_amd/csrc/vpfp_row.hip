@@ -40,9 +40,9 @@ int launch_row_q(const vp::RowArgs<T>& a, hipStream_t s) {
 //   FP32 M = 4096: one workgroup of 512 threads fits a CU, or two of 256.  With
 //     more rows than CUs 16: 1024 rows 469 -> 366 us, 512 rows 284 -> 239 (256
 //     rows 165 and 168); delta-f 561 -> 438 and 328 -> 272.  No less accurate: f
-//     after four steps with collisions 6.6e-7 and 5.9e-7 off, without 7.1e-7 and
-//     5.8e-7, delta-f 7.6e-7 and 7.1e-7; E 4.7e-7 and 4.6e-7, 4.6e-7 and 4.0e-7,
-//     1.7e-7 and 1.6e-7 (means over 8 initial states).
+//     after four steps with collisions 6.4e-7 and 5.7e-7 off, without 6.9e-7 and
+//     5.7e-7, delta-f 7.2e-7 and 6.6e-7; E 4.8e-7 and 4.6e-7, 4.4e-7 and 3.3e-7,
+//     1.4e-7 and 1.3e-7 (means over 8 initial states).
 //   FP32 M = 2048: 8.  16 take 250 -> 229 us at 1024 rows, 409 -> 401 at 2048, but
 //     lose at 512 (154, 163) and with delta-f (2048 rows 475, 545).
 //   FP64: 8 (M = 4096 at 16 values spills 260 bytes at two workgroups per CU:
